@@ -1,0 +1,457 @@
+"""Performance cases: the work a user of approxtorch_amd has it do.
+
+Each case is one pass through a public entry point (a quantized conv layer's
+forward, or its forward and backward; a LUT GEMM op; a whole training step of
+a converted network) on inputs that are in GPU memory, as they are in a
+training or inference program.  `listed()` gives the fixed cases, `draw()`
+more of the same ranges.
+
+The layers run with scale_momentum 1.0, so a training pass leaves the EMA
+statistics at the batch's own values and every pass of one state does the
+same work with the same result.
+"""
+import functools
+import math
+
+import numpy as np
+import torch
+import torch.nn.functional as F
+
+import approxtorch_amd as at
+from approxtorch_amd import workloads
+from approxtorch_amd.backend import ops
+from approxtorch_amd.nn import bgemm_int8
+
+DEV = "cuda"
+
+
+def _conv(name, **kw):
+    case = dict(name=name, kind="conv", qtype="int8", grad="lre", bits=8, lut="perturbed",
+                train=True, n=64, c=64, o=64, kh=3, kw=3, stride=1, pad=1, dil=1, h=28, w=28,
+                bias=False, signed=False, depthwise=False, dtype="float32")
+    case.update(kw)
+    return case
+
+
+def listed():
+    return [
+        # one layer of a served model, a small batch: launches and host issue count
+        _conv("eval_small", train=False, grad="ste", lut="exact", n=8, h=32, w=32),
+        # ResNet-50 at 224 x 224, batch 64: the first stage's 3x3 convs
+        _conv("train_3x3_56", h=56, w=56),
+        # a later stage's 1x1 reduction: long contraction, few rows
+        _conv("train_1x1_14", c=1024, o=256, kh=1, kw=1, pad=0, h=14, w=14),
+        # the strided 3x3 conv between two stages
+        _conv("train_s2_56", c=128, o=128, stride=2, h=56, w=56),
+        # a user's own network: odd sizes, signed inputs (no ReLU before), bias,
+        # rectangular kernel, autocast's bf16 activations
+        _conv("train_odd_bf16", grad="ste", lut="trunc4", n=19, c=45, o=83, kh=5, kw=3, pad=2,
+              h=29, w=23, bias=True, signed=True, dtype="bfloat16"),
+        # MobileNetV2's depthwise convs
+        _conv("train_depthwise", n=64, c=144, o=144, h=56, w=56, depthwise=True),
+        # ResNet-50 with 4-bit uint8 weights and pair-table gradients, batch 128
+        _conv("train_u8w4_3x3_28", qtype="uint8", grad="custom", bits=4, lut="u16mask", n=128,
+              c=128, o=128),
+        # its last stage: 7 x 7 images (rows not a multiple of 4)
+        _conv("train_u8w4_1x1_7", qtype="uint8", grad="custom", bits=4, lut="u16mask", n=128,
+              c=2048, o=512, kh=1, kw=1, pad=0, h=7, w=7),
+        # the uint8 layer's default weight width with pair-table gradients
+        _conv("train_u8_custom_14", qtype="uint8", grad="custom", lut="u16mask", n=32, c=128,
+              o=128, h=14, w=14, bias=True),
+        # the LUT BGEMM op under autograd (straight-through), conv-shaped operands
+        dict(name="bgemm_ste", kind="bgemm", n=16, k=1152, l=784, o=128, lut="perturbed"),
+        # an approximate linear layer's product on a ragged token count
+        dict(name="gemm_linear", kind="gemm", m=1000, n=4096, k=1024, lut="perturbed"),
+        # a whole training step: ResNet-18 for 32 x 32 images, batch 128
+        dict(name="resnet18_step", kind="resnet18", n=128, lut="trunc4"),
+    ]
+
+
+def _logint(rng, lo, hi):
+    return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+
+def draw(rng):
+    kind = rng.choice(["int8", "int8", "int8", "int8", "eval", "depthwise", "u8w4", "u8w4", "u8",
+                       "bgemm", "gemm", "resnet18"])
+    if kind == "resnet18":
+        return dict(kind="resnet18", n=_logint(rng, 4, 128), lut="trunc4")
+    while True:
+        if kind == "bgemm":
+            case = dict(kind="bgemm", n=_logint(rng, 1, 64), k=_logint(rng, 27, 4608),
+                        l=_logint(rng, 16, 3136), o=_logint(rng, 16, 512),
+                        lut=rng.choice(["perturbed", "trunc4"]))
+            macs = case["n"] * case["k"] * case["l"] * case["o"]
+            if 1e7 <= macs <= 8e9:
+                return case
+            continue
+        if kind == "gemm":
+            case = dict(kind="gemm", m=_logint(rng, 1, 8192), n=_logint(rng, 64, 8192),
+                        k=_logint(rng, 64, 8192), lut=rng.choice(["perturbed", "trunc4"]))
+            if 1e6 <= case["m"] * case["n"] * case["k"] <= 1.5e10:
+                return case
+            continue
+        k = rng.choice([1, 1, 3, 3, 3, 5])
+        case = _conv("", n=_logint(rng, 1, 128), c=_logint(rng, 3, 1024), o=_logint(rng, 8, 1024),
+                     kh=k, kw=k, stride=rng.choice([1, 1, 1, 2]), pad=k // 2,
+                     dil=rng.choice([1, 1, 1, 2]) if k > 1 else 1,
+                     h=_logint(rng, 5, 64), w=0, bias=rng.random() < 0.3,
+                     signed=rng.random() < 0.3)
+        case.pop("name")
+        case["w"] = case["h"] if rng.random() < 0.7 else _logint(rng, 5, 64)
+        case["pad"] *= case["dil"]
+        limit = 1.5e10
+        if kind == "int8" or kind == "eval":
+            case.update(grad=rng.choice(["ste", "lre"]), train=kind == "int8",
+                        lut=rng.choice(["exact", "trunc4", "perturbed"]),
+                        bits=rng.choice([8, 8, 8, 8, 6, 4]),
+                        dtype=rng.choice(["float32", "float32", "float32", "bfloat16"]))
+        elif kind == "depthwise":
+            case.update(depthwise=True, o=case["c"], kh=3, kw=3, pad=case["dil"],
+                        grad=rng.choice(["ste", "lre"]))
+        else:
+            case.update(qtype="uint8", grad="custom", lut="u16mask", dil=1, pad=k // 2,
+                        bits=4 if kind == "u8w4" else 8)
+            if kind == "u8":
+                case["grad"] = rng.choice(["custom", "custom", "lre", "ste"])
+                limit = 2e9
+        if 1e6 <= _macs(case) <= limit and _elems(case) <= 4e7:
+            return case
+
+
+# ------------------------------------------------------------------ sizes
+def _out_hw(case):
+    eh = case["dil"] * (case["kh"] - 1) + 1
+    ew = case["dil"] * (case["kw"] - 1) + 1
+    return ((case["h"] + 2 * case["pad"] - eh) // case["stride"] + 1,
+            (case["w"] + 2 * case["pad"] - ew) // case["stride"] + 1)
+
+
+def _taps(case):
+    return case["kh"] * case["kw"] * (1 if case["depthwise"] else case["c"])
+
+
+def _macs(case):
+    oh, ow = _out_hw(case)
+    return case["n"] * oh * ow * case["o"] * _taps(case)
+
+
+def _elems(case):
+    oh, ow = _out_hw(case)
+    return case["n"] * max(case["c"] * case["h"] * case["w"], case["o"] * oh * ow)
+
+
+RESNET18_MACS = 553_648_128        # converted convs of one 32 x 32 image
+
+
+def work(case):
+    """Two operations per product; the backward adds one product per forward
+    product for each of its two gradients."""
+    if case["kind"] == "bgemm":
+        n, k, l, o = case["n"], case["k"], case["l"], case["o"]
+        return {"bytes": 4 * (2 * n * k * l + 2 * o * k + 2 * n * o * l) + 4 * 65536,
+                "flops": 6 * n * k * l * o}
+    if case["kind"] == "gemm":
+        m, n, k = case["m"], case["n"], case["k"]
+        return {"bytes": 4 * (m * k + n * k + m * n) + 4 * 65536, "flops": 2 * m * n * k}
+    if case["kind"] == "resnet18":
+        # each conv's input and output once forward, once backward (11.2 M weights)
+        return {"bytes": case["n"] * 4 * 2_900_000 + 11_200_000 * 4 * 2,
+                "flops": 6 * case["n"] * RESNET18_MACS}
+    oh, ow = _out_hw(case)
+    item = 2 if case["dtype"] == "bfloat16" else 4
+    x = case["n"] * case["c"] * case["h"] * case["w"] * item
+    y = case["n"] * case["o"] * oh * ow * 4
+    w = case["o"] * _taps(case) * 4
+    tables = 4 * 65536
+    if not case["train"]:
+        return {"bytes": x + w + y + tables, "flops": 2 * _macs(case)}
+    tables += 2 * 4 * (65536 if case["grad"] == "custom" else 256)
+    return {"bytes": 2 * x + 2 * y + 2 * w + tables, "flops": 6 * _macs(case)}
+
+
+# ----------------------------------------------------------------- tables
+@functools.lru_cache(maxsize=None)
+def _lut(name):
+    make = {"exact": workloads.lut_exact_int8, "trunc4": workloads.lut_trunc4,
+            "perturbed": workloads.lut_perturbed, "u16mask": workloads.lut_u16mask}[name]
+    return torch.from_numpy(np.ascontiguousarray(make()))
+
+
+@functools.lru_cache(maxsize=None)
+def _grad_tables(lut, grad, qtype):
+    if grad == "ste":
+        return None, None
+    if grad == "lre":
+        return workloads.lre_tables(_lut(lut).numpy(), qtype)
+    return workloads.date_tables(_lut(lut).numpy(), 2)
+
+
+# ----------------------------------------------------------------- inputs
+def _generator(seed):
+    return torch.Generator(device=DEV).manual_seed(seed)
+
+
+def _conv_inputs(case, seed):
+    """x (ReLU outputs, or signed), weight, bias, output gradient."""
+    g = _generator(seed)
+    oh, ow = _out_hw(case)
+
+    def randn(*shape):
+        return torch.randn(shape, generator=g, device=DEV)
+    x = randn(case["n"], case["c"], case["h"], case["w"])
+    if not case["signed"]:
+        x = x.relu_()
+    x = x.to(getattr(torch, case["dtype"]))
+    taps = _taps(case)
+    wt = randn(case["o"], taps // (case["kh"] * case["kw"]), case["kh"], case["kw"])
+    wt = wt * math.sqrt(2.0 / taps)
+    b = randn(case["o"]) * 0.1 if case["bias"] else None
+    go = randn(case["n"], case["o"], oh, ow) * 1e-3
+    return x, wt, b, go
+
+
+def _quantized(shape, g):
+    return torch.randint(-127, 128, shape, generator=g, device=DEV).float()
+
+
+def _bgemm_inputs(case, seed):
+    g = _generator(seed)
+    x = _quantized((case["n"], case["k"], case["l"]), g)
+    w = _quantized((case["o"], case["k"]), g)
+    go = torch.randn((case["n"], case["o"], case["l"]), generator=g, device=DEV) * 1e-3
+    return x, w, go
+
+
+def _gemm_inputs(case, seed):
+    g = _generator(seed)
+    a = _quantized((case["m"], case["k"]), g)
+    b = _quantized((case["n"], case["k"]), g)      # a linear layer's weight
+    return a, b
+
+
+def prepare(case, seed):
+    lut = _lut(case["lut"]).to(DEV)
+    if case["kind"] == "bgemm":
+        x, w, go = _bgemm_inputs(case, seed)
+        return dict(case=case, x=x.requires_grad_(), w=w.requires_grad_(), go=go, lut=lut)
+    if case["kind"] == "gemm":
+        a, b = _gemm_inputs(case, seed)
+        return dict(case=case, a=a, b=b.t(), lut=lut)
+    if case["kind"] == "resnet18":
+        with torch.random.fork_rng(devices=[torch.cuda.current_device()]):
+            torch.manual_seed(seed)
+            model = workloads.resnet18_cifar(10)
+        model = at.convert_model(model, lut, qtype="int8", grad="ste", scale_momentum=1.0)
+        model = model.to(DEV).train()
+        g = _generator(seed)
+        x = torch.randn((case["n"], 3, 32, 32), generator=g, device=DEV)
+        y = torch.randint(0, 10, (case["n"],), generator=g, device=DEV)
+        return dict(case=case, model=model, x=x, y=y, params=list(model.parameters()))
+    x, wt, b, go = _conv_inputs(case, seed)
+    dx, dw = _grad_tables(case["lut"], case["grad"], case["qtype"])
+    cls = at.nn.Conv2d_int8 if case["qtype"] == "int8" else at.nn.Conv2d_uint8
+    layer = cls(case["c"], case["o"], (case["kh"], case["kw"]), lut, grad=case["grad"],
+                dx=None if dx is None else dx.to(DEV), dw=None if dw is None else dw.to(DEV),
+                bias=case["bias"], stride=case["stride"], padding=case["pad"],
+                dilation=case["dil"], groups=case["c"] if case["depthwise"] else 1,
+                scale_momentum=1.0, weight_bits=case["bits"]).to(DEV)
+    with torch.no_grad():
+        layer.weight.copy_(wt)
+        if b is not None:
+            layer.bias.copy_(b)
+    layer.train()
+    if not case["train"]:
+        with torch.no_grad():
+            layer(x)               # the statistics a calibrated model holds
+        layer.eval()
+        return dict(case=case, layer=layer, x=x)
+    params = [x.requires_grad_(), layer.weight] + ([layer.bias] if case["bias"] else [])
+    return dict(case=case, layer=layer, x=x, go=go, params=params)
+
+
+def run(state):
+    case = state["case"]
+    if case["kind"] == "bgemm":
+        y = bgemm_int8.bgemm_int8_ste(state["x"], state["w"], state["lut"])
+        return (y,) + torch.autograd.grad(y, [state["x"], state["w"]], state["go"])
+    if case["kind"] == "gemm":
+        return ops.gemm_fake_int8_claude(state["a"], state["b"], state["lut"])
+    if case["kind"] == "resnet18":
+        logits = state["model"](state["x"])
+        loss = F.cross_entropy(logits, state["y"])
+        return (logits,) + torch.autograd.grad(loss, state["params"])
+    if not case["train"]:
+        with torch.no_grad():
+            return state["layer"](state["x"])
+    y = state["layer"](state["x"])
+    return (y,) + torch.autograd.grad(y, state["params"], state["go"])
+
+
+# -------------------------------------------------------------- tolerance
+def tolerance(case):
+    """About four times the error of the outputs against `exact` (measured over
+    the listed and twenty drawn cases).  Integer sums converted to fp32 are
+    exact to half an ulp."""
+    if case["kind"] == "gemm":
+        return {"rel": 2e-7}
+    if case["kind"] == "bgemm":
+        return {"rel": 4e-6}
+    if case["kind"] == "resnet18":
+        # the forward's sums are integers, so its values stay the same bits; the
+        # gradients' fp32 sums in another order, carried through nineteen layers
+        return {"rel": 2e-4}
+    if not case["train"]:
+        return {"rel": 1e-6}
+    if case["dtype"] == "bfloat16":
+        return {"rel": 8e-3}       # grad_x is rounded to bf16
+    return {"rel": 4e-6}
+
+
+# ------------------------------------------------------------------ exact
+# Sums, products and gradients in 64 bits.  The quantized values themselves
+# are the layer's definition (round(x / scale) of fp32 or bf16 statements) and
+# are taken from those statements.
+def _lut_rows(table, idx_x, idx_w):
+    """table[idx_x, idx_w[o]] for every row: [rows, O] (idx_x [rows])."""
+    return table[:, idx_w][idx_x]
+
+
+def _unfold(img, case, pad_value):
+    """[N, K, L] of an image padded with pad_value (exact for small integers)."""
+    p = case["pad"]
+    padded = F.pad(img, (p, p, p, p), value=float(pad_value))
+    return F.unfold(padded, (case["kh"], case["kw"]), dilation=case["dil"],
+                    stride=case["stride"])
+
+
+def _fold(col, case):
+    return F.fold(col, (case["h"], case["w"]), (case["kh"], case["kw"]), dilation=case["dil"],
+                  padding=case["pad"], stride=case["stride"])
+
+
+def _quantize(case, x, wt):
+    """(qx, mask_x, scale_x, zero_x, qw, mask_w, scale_w, zero_w) as the layer
+    defines them with statistics of this batch."""
+    w = wt.reshape(case["o"], -1)
+    if case["qtype"] == "int8":
+        qmax_w = 2 ** (case["bits"] - 1) - 1
+        sx = x.abs().max() / 127
+        sw = w.abs().amax(1) / qmax_w
+        v = x / sx.to(x.dtype)
+        vw = w / sw.view(-1, 1)
+        zx, zw = sx.new_zeros((), dtype=torch.float32), torch.zeros_like(sw)
+        lo_x, hi_x, lo_w, hi_w = -127, 127, -qmax_w, qmax_w
+    else:
+        hi_w = 2 ** case["bits"] - 1
+
+        def qparams(mn, mx, top):
+            mn, mx = mn.clamp(max=0.0), mx.clamp(min=0.0)
+            s = ((mx - mn) / top).clamp(min=1e-12)
+            return s, torch.round(-mn / s).clamp(0.0, float(top))
+        sx, zx = qparams(x.min(), x.max(), 255)
+        sw, zw = qparams(w.amin(1), w.amax(1), hi_w)
+        v = x / sx + zx
+        vw = w / sw.view(-1, 1) + zw.view(-1, 1)
+        lo_x, hi_x, lo_w = 0, 255, 0
+    qx, mx = torch.round(v).clamp(lo_x, hi_x).float(), (v >= lo_x) & (v <= hi_x)
+    qw, mw = torch.round(vw).clamp(lo_w, hi_w), (vw >= lo_w) & (vw <= hi_w)
+    return qx, mx, sx.double(), zx.double(), qw, mw, sw.double(), zw.double()
+
+
+def _exact_conv(case, seed):
+    x, wt, b, go = _conv_inputs(case, seed)
+    qx, mx, sx, zx, qw, mw, sw, zw = _quantize(case, x, wt)
+    lut = _lut(case["lut"]).to(DEV).double().view(256, 256)
+    off = 128 if case["qtype"] == "int8" else 0
+    n, o, taps = case["n"], case["o"], _taps(case)
+    oh, ow = _out_hw(case)
+    length = oh * ow
+    xu = _unfold(qx, case, float(zx)).add_(off)             # [N, C*KH*KW, L] indices
+    wi = qw.long() + off                                    # [O, K]
+    dx, dw = _grad_tables(case["lut"], case["grad"], case["qtype"])
+    ident = torch.arange(256, device=DEV, dtype=torch.float64) - off
+    if case["grad"] == "ste":
+        dx = dw = ident
+    else:
+        dx, dw = dx.to(DEV).double(), dw.to(DEV).double()
+    scale = sx * sw
+    g2 = go.double().view(n, o, length) * scale.view(1, -1, 1)
+    if case["depthwise"]:
+        xi = xu.view(n, o, taps, length).long()
+        y = torch.zeros((n, o, length), dtype=torch.float64, device=DEV)
+        gcol = torch.empty((n, o, taps, length), dtype=torch.float64, device=DEV)
+        gw = torch.empty((o, taps), dtype=torch.float64, device=DEV)
+        for t in range(taps):
+            y += lut.view(-1)[xi[:, :, t] * 256 + wi[:, t].view(1, -1, 1)]
+            gcol[:, :, t] = g2 * dx[wi[:, t]].view(1, -1, 1)
+            gw[:, t] = (g2 * dw[xi[:, :, t]]).sum((0, 2))
+        gcol = gcol.view(n, o * taps, length)
+    else:
+        rows = g2.permute(0, 2, 1).reshape(n * length, o)   # output gradient by row
+        y = torch.zeros((n * length, o), dtype=torch.float64, device=DEV)
+        pair = case["grad"] == "custom" and case["train"]
+        if pair:
+            dx, dw = dx.view(256, 256), dw.view(256, 256)
+            gcol = torch.empty((n, taps, length), dtype=torch.float64, device=DEV)
+            gw = torch.empty((o, taps), dtype=torch.float64, device=DEV)
+        for k in range(taps):
+            idx = xu[:, k].reshape(-1).long()
+            y += _lut_rows(lut, idx, wi[:, k])
+            if pair:
+                gcol[:, k] = (_lut_rows(dx, idx, wi[:, k]) * rows).sum(1).view(n, length)
+                gw[:, k] = (_lut_rows(dw, idx, wi[:, k]) * rows).sum(0)
+        if case["train"] and not pair:
+            wtab = dx[wi].t().contiguous()                  # [K, O]
+            gcol = (rows @ wtab.t().contiguous()).view(n, length, taps)
+            gcol = gcol.permute(0, 2, 1).contiguous()
+            gw = torch.zeros((o, taps), dtype=torch.float64, device=DEV)
+            for i in range(n):
+                gw += g2[i] @ dw[xu[i].long()].t().contiguous()
+        y = y.view(n, length, o).permute(0, 2, 1)
+    if case["qtype"] == "uint8":
+        xs = xu.double().sum(1)
+        ws = wi.double().sum(1)
+        y = y - zw.view(1, -1, 1) * xs.unsqueeze(1) - (zx * ws).view(1, -1, 1) + \
+            (taps * zx * zw).view(1, -1, 1)
+        if case["train"]:
+            gcol -= (g2 * zw.view(1, -1, 1)).sum(1, keepdim=True)
+            gw -= zx * g2.sum((0, 2)).view(-1, 1)
+    y = y * scale.view(1, -1, 1)
+    if b is not None:
+        y = y + b.double().view(1, -1, 1)
+    y = y.reshape(n, o, oh, ow)
+    if not case["train"]:
+        return y
+    gx = torch.where(mx, _fold(gcol, case), 0.0) / sx
+    gw = torch.where(mw, gw, 0.0) / sw.view(-1, 1)
+    out = (y, gx, gw.view(wt.shape))
+    return out + ((go.double().sum((0, 2, 3)),) if b is not None else ())
+
+
+def exact(case, seed):
+    if case["kind"] == "resnet18":
+        return None         # a value next to a quantization step has no such result
+    if case["kind"] == "conv":
+        return _exact_conv(case, seed)
+    lut = _lut(case["lut"]).to(DEV).double().view(256, 256)
+    if case["kind"] == "gemm":
+        a, b = _gemm_inputs(case, seed)
+        y = torch.zeros((case["m"], case["n"]), dtype=torch.float64, device=DEV)
+        a, b = a.long() + 128, b.long() + 128
+        for k in range(case["k"]):
+            y += _lut_rows(lut, a[:, k], b[:, k])
+        return y
+    x, w, go = _bgemm_inputs(case, seed)
+    n, k, l, o = case["n"], case["k"], case["l"], case["o"]
+    y = torch.zeros((n * l, o), dtype=torch.float64, device=DEV)
+    wi = w.long() + 128
+    for t in range(k):
+        y += _lut_rows(lut, x[:, t].reshape(-1).long() + 128, wi[:, t])
+    gx = torch.empty((n, k, l), dtype=torch.float64, device=DEV)
+    gw = torch.zeros((o, k), dtype=torch.float64, device=DEV)
+    wd = w.double().t().contiguous()
+    for i in range(n):
+        gx[i] = wd @ go[i].double()
+        gw += go[i].double() @ x[i].double().t().contiguous()
+    return y.view(n, l, o).permute(0, 2, 1).contiguous(), gx, gw
