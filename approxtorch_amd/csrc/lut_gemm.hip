@@ -1,47 +1,60 @@
 // LUT GEMM forward for gfx950: y[n,o,l] = sum_k LUT[xi(n,k,l)][wi(o,k)].
 //
-// Kernel structure ("expanded tables", four to an LDS line):
+// Kernel structure ("expanded tables" in byte planes, added by the matrix
+// cores):
 //   A workgroup owns a tile of ATX_ROW_TILE (2048) rows r = n*L + l and
 //   ATX_COL_TILE (32) output channels.  For every k it builds, in LDS, the
-//   table E_k[v][o] = LUT16[v][wi(o,k)] (256 rows x 32 channels x 16 bit =
-//   16 KiB) from the transposed 16-bit LUT image (L2-resident, 128 KiB), then
-//   every lane looks up E_k[xi(r,k)][o..o+7] for its rows with one 16-byte
-//   LDS read and adds the eight 16-bit entries into int32 accumulators
-//   (exact).  Table bytes written per lookup are 512 / ATX_ROW_TILE, so the
-//   tall, narrow tile halves the table-build cost of a 1024 x 64 tile with
-//   the same accumulators per lane.
+//   table E_k[v][o] = LUT16[v][wi(o,k)] (256 rows x 32 channels) from the
+//   transposed 16-bit LUT image (L2-resident, 128 KiB), each row as two
+//   16-channel chunks of high bytes and two of low bytes.  A lane looks a
+//   row's 16 channels up with two 16-byte LDS reads, and one sparse matrix
+//   product (v_smfmac_i32_16x16x128_i8) adds them: its 4:2-sparse operand is a
+//   fixed selection matrix (row i picks byte i of every chunk, weighted by the
+//   plane), so 64 lanes' 32 bytes - 16 rows x 4 taps x 16 channels x 2 planes
+//   - go into 16 x 16 int32 sums.  The high plane's weight 256 does not fit an
+//   int8, so a second product adds the high bytes once more (-128 each).
 //
-//   LDS bank layout.  gfx950's LDS has 64 banks (256 bytes per clock) and
-//   serves a 16-byte read in passes of 16 lanes.  An E row is 64 bytes, so a
-//   pass covers four rows, and rows landing in the same quarter of the banks
-//   serialize.  Four consecutive tables therefore share each 256-byte LDS
-//   line: line v holds row v of table 4j+q in quarter q.  In sub-step s of
-//   quad j, row group rg reads table 4j + ((rg + s) & 3); the four row
-//   groups of a pass read four different quarters whatever their rows, so
-//   the reads are conflict-free (130 TB/s measured, against 66 TB/s for
-//   random quarters).  Over the quad's four sub-steps every lane reads all
-//   four tables.  Within a quarter, the 16-byte chunk for channels 8g..8g+7
-//   of row v sits at position g ^ ((v >> 1) & 3).  The activation operand is
-//   pre-encoded as the byte offset v*256 + ((v >> 1) & 3)*16 ("row offset");
-//   a lane's address is row_offset ^ (g*16 | quarter*64 | buffer*65536).
+//   What bounds it: the LDS reads (2 bytes per lookup; conflict-free 16-byte
+//   reads measure 122 TB/s = 61 T lookups/s), then the table build.  Reads
+//   plus both products measure 44-46 T lookups/s; with one VALU add per
+//   lookup in their place (packed pairs, 1.26 VALU instructions per lookup)
+//   the same loop measured 30.7 T.  Whole kernel, K = 2304, 65536 rows x 64
+//   channels: 537 -> 406 us with upper-half tables (24 T), 558 -> 441 us with
+//   full ones; K = 1024, 12544 x 256: 201 -> 145 us; K = 64, 200704 x 256: 222
+//   -> 167 us.  Timed copies (100352 x 128, K = 1152, full tables, 650 us):
+//   without the LUT-row loads 505, without the table writes as well 410.  The
+//   LUT rows (64 KiB per quad from L1 / L2 at 64 bytes a clock) and the LDS
+//   reads do not overlap fully; that is what is left.
 //
-//   Table build: two quad buffers (128 KiB).  In sub-step s of quad j every
-//   wave writes its part of table 4(j+1)+s into the other buffer: wave w
-//   covers channel group w % 4 for rows 128(w / 4) .. +127; its eight
-//   weight indices are wave-uniform (one vector load read back with
-//   v_readlane); lane t loads the dwords LUT16T[w_c][v0, v0+1] (v0 = row
-//   pair of the lane) of the eight channels c (buffer loads, scalar offsets),
-//   interleaves them with v_perm into the 16-byte chunks of rows v0 and v0+1
-//   and stores each with one ds_write_b128.  One barrier per quad (four
-//   k-steps) orders the build of quad j+1 and the reads of quad j.
+//   LDS layout.  gfx950's LDS has 64 banks (256 bytes per clock); it serves a
+//   16-byte read in passes of 16 lanes, 0-3, 12-15 and 20-27 the first, then
+//   4-11, 16-19 and 28-31, and the same of the upper half.  Four consecutive
+//   tables share each 256-byte line: line v holds row v of tap t in quarter t
+//   (channel half cg at + 32, plane at + 16; 0 = high).  Lane (j, g) = (lane &
+//   15, lane >> 4) reads tap (j & 3) ^ g, channel half (j >> 3) ^ c and plane
+//   (g & 1) ^ h in its read (c, h): the lanes of a pass read sixteen different
+//   positions of a line, whatever their rows, so no two share a bank.  The
+//   activation operand is pre-encoded as the byte offset v*256 + ((v >> 1) &
+//   3)*16 ("row offset"), of which this kernel takes the byte v: one v_perm
+//   puts it above the lane's position bits.
 //
-//   Threads: 512 (8 waves).  Lane = (row group rg 0..15, channel group g);
-//   wave w owns rows 256w .. 256w+255 of the tile and lane (rg, g) the rows
-//   64h + 4rg + m (h, m = 0..3) x 8 channels = 128 int32 accumulators
-//   (256-VGPR budget at 2 waves per SIMD).  Four consecutive rows per lane
-//   let the epilogue store every (channel, h) as one 16-byte vector, and the
-//   sixteen row groups of a channel fill two 128-byte lines, so results go
-//   from registers straight to HBM with all waves storing at once.
+//   Table build: two quad buffers (128 KiB).  While quad j is read, the wave
+//   transposes its share of quad j+1 (entries loaded during quad j-1) with
+//   v_perm into chunks, stores them, and then loads the entries of quad j+2,
+//   one channel per two reads: a burst of sixteen loads at one place stalled
+//   the wave's reads behind the address unit (c. 15% of the kernel).  A wave
+//   builds one tap; its lanes cover 128 consecutive rows of both channel
+//   halves, so a load instruction touches two LUT rows (eight rows of 64 bytes
+//   each measured twice the time), and the four lanes of a store pass write
+//   four different positions (two halves, planes in the order of lane bit 0).
+//   One barrier per quad (four k-steps) orders build and reads.
+//
+//   Threads: 512 (8 waves, 2 per SIMD).  Wave w owns rows 256w .. 256w+255 of
+//   the tile; lane (j, g) the rows 64h + 4j + m (h, m = 0..3) x 8 channels =
+//   128 int32 accumulators of its 256 registers.  Four consecutive rows per
+//   lane let the epilogue store every (channel, h) as one 16-byte vector,
+//   eight lanes one 128-byte line (sixteen consecutive rows per lane, 16-byte
+//   pieces 64 bytes apart, measured 10-40% slower).
 //
 // Reference: bgemm_lut_u8_kernel / bgemm_mainloop
 // (csrc/claude/bgemm_lut_kernels.cuh:183-387) computes the same sum with a
@@ -60,12 +73,8 @@ namespace atx {
 
 constexpr int RT = ATX_ROW_TILE;   // rows per workgroup (2048)
 constexpr int OT = ATX_COL_TILE;   // channels per workgroup (32)
-constexpr int CG = OT / 8;         // 16-byte channel chunks per table row (4)
-constexpr int NRG = 64 / CG;       // row groups per wave (16)
-constexpr int RQ = 4;              // consecutive rows per lane quad
-constexpr int NQ = 4;              // quads per lane (stride NRG * RQ rows)
-constexpr int RPL = RQ * NQ;       // rows per lane (16)
-constexpr int RPW = NRG * RPL;     // rows per wave (256)
+constexpr int RPL = 16;            // rows per lane
+constexpr int RPW = 16 * RPL;      // rows per wave (256)
 constexpr int NWAVE = RT / RPW;    // waves per workgroup (8)
 constexpr int NT = 64 * NWAVE;     // threads per workgroup (512)
 constexpr int TPL = 4;             // tables per LDS line (quarters)
@@ -73,10 +82,8 @@ constexpr int LINE = 256;          // bytes per LDS line
 constexpr int QTAB = 256 * LINE;   // one quad of tables (64 KiB)
 constexpr int SMEM_BYTES = 2 * QTAB;          // two quad buffers (128 KiB)
 static_assert(QTAB == 1 << 16, "quad buffer select is bit 16 of a read address");
-static_assert(CG == 4 && NRG == 16 && NWAVE == 8, "tile geometry");
-static_assert(TPL * CG * 16 == LINE, "four 64-byte table rows per line");
-static_assert(2 * NWAVE == 16 && 256 / 2 == 64 * (NWAVE / CG),
-              "a table is 8 waves x 64 lanes x one row pair");
+static_assert(OT == 32 && NWAVE == 8, "tile geometry");
+static_assert(TPL * OT * 2 == LINE, "four 64-byte table rows per line");
 
 // K limits for exact int32 partial sums (entries up to 32767 / 65535).
 constexpr int KMAX_I16 = 65536;
@@ -110,6 +117,7 @@ struct GemmParams {
   // below R is at least 128 (x >= 0 before an int8 fake-quant).  The tables
   // are then built for rows 128..255 only (upper-half tables).
   const int* x_upper;
+  bool sgn;                     // signed (int16) table entries
 };
 
 // ------------------------------------------------------------------ prepare
@@ -343,338 +351,324 @@ __global__ void pack_w_kernel(const T* __restrict__ w, int O, int K, int offset,
 }
 
 // ------------------------------------------------------------- main kernel
-// Accumulates one 16-byte table chunk (channels 2m, 2m+1 in dword m, the
-// even channel in the low half) into a row's pair accumulators:
-// a[2m] += d_m, the whole dword, and a[2m+1] += d_m >> 16, the high entry
-// (sign-extended for signed tables).  The even channels' sums are recovered
-// once per tile segment (pair_sums): a[2m] - (a[2m+1] << 16), less the bias
-// of the low entries for signed tables.  One add of each pair is a plain
-// 32-bit VOP2 add, which gfx950 issues at about 1.7x the rate of the SDWA
-// form that extracts a 16-bit half.
-template <bool SIGNED>
-__device__ __forceinline__ void add8(int (&a)[8], const uint4 e) {
-  const unsigned d[4] = {e.x, e.y, e.z, e.w};
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    a[2 * i] = (int)((unsigned)a[2 * i] + d[i]);
-    if constexpr (SIGNED) a[2 * i + 1] += ((int)d[i]) >> 16;
-    else a[2 * i + 1] += (int)(d[i] >> 16);
-  }
+using v4i = int __attribute__((ext_vector_type(4)));
+using v8i = int __attribute__((ext_vector_type(8)));
+
+constexpr int RD = 4;              // table reads (32-byte pairs) in flight per lane
+static_assert(8 % RD == 0, "a row quad's reload follows a whole ring");
+
+// The lane's accumulators: acc[4 h + m][c][q] is row 64 h + 4 j + m of the
+// wave, channel 16 ((j >> 3) ^ c) + 4 g + q of the tile (j = lane & 15, g =
+// lane >> 4).
+using Acc = v4i[RPL][2];
+
+// Selection operand of the sparse matrix product (16 x 128, 4:2 sparse):
+// row i has one entry in each of the 16-byte chunks a lane group reads, at
+// byte i, so the product adds, for every channel i, the chunks' bytes i of
+// the four lane groups.  The weights undo the byte split: a high byte counts
+// -256 (two products of -128: an int8 holds no 256) and a low byte -1.
+// Lane group g and register half h of the table operand hold plane
+// (g & 1) ^ h (0 high, 1 low).  In the instruction's layout lane group ga of
+// this operand covers half ga >> 1, lane group 2 (ga & 1) in its bytes 0-7
+// and 2 (ga & 1) + 1 in bytes 8-15; a group of four k has two value slots,
+// whose positions are in idx.
+struct Select { v4i both, high; int idx; };
+
+__device__ __forceinline__ Select make_select(int lane) {
+  const int i = lane & 15, half = lane >> 5, pos = i & 3;
+  const int shift = 8 * (2 * ((i >> 2) & 1) + (pos == 3));
+  const unsigned hi = 0x80u << shift;                   // -128
+  const unsigned lo = 0xffu << shift;                   // -1
+  const unsigned b0 = half ? lo : hi, b1 = half ? hi : lo;
+  const unsigned h0 = half ? 0u : hi, h1 = half ? hi : 0u;
+  const bool up = (i >> 3) != 0;
+  Select s;
+  s.both = v4i{up ? 0 : (int)b0, up ? (int)b0 : 0, up ? 0 : (int)b1, up ? (int)b1 : 0};
+  s.high = v4i{up ? 0 : (int)h0, up ? (int)h0 : 0, up ? 0 : (int)h1, up ? (int)h1 : 0};
+  s.idx = (int)(((pos < 3 ? (unsigned)pos : 0u) | 12u) * 0x11111111u);
+  return s;
 }
 
-// Signed tables store their low (even-channel) entries biased by 2^15, so
-// that a dword's value is exactly hi * 2^16 + (lo + 2^15) with the low part
-// in [0, 2^16): summed over T tables, the even channel's sum is
-// S - (H << 16) - 2^15 T (mod 2^32; exact within the int32 bound).
-constexpr unsigned LOW_BIAS = 0x8000u;
+// Byte code of a table entry: the 16-bit entry with its low byte (and, for
+// unsigned tables, its high byte) offset to a signed byte.  Summed with the
+// weights above T entries give -(sum - code_bias T).
+__device__ __forceinline__ unsigned code_xor(bool sgn) { return sgn ? 0x00800080u : 0x80808080u; }
+__device__ __forceinline__ int code_bias(bool sgn) { return sgn ? 128 : 32768 + 128; }
 
-// Turns the pair accumulators of the lane's rows into channel sums after
-// `tables` tables (every table accumulated, all-zero ones included: their
-// biased low entries are exactly LOW_BIAS).
-template <bool SIGNED>
-__device__ __forceinline__ void pair_sums(int (&acc)[RPL][8], int tables) {
-  const unsigned bias = SIGNED ? LOW_BIAS * (unsigned)tables : 0u;
-#pragma unroll
-  for (int j = 0; j < RPL; ++j)
-#pragma unroll
-    for (int m = 0; m < 4; ++m)
-      acc[j][2 * m] =
-          (int)((unsigned)acc[j][2 * m] - ((unsigned)acc[j][2 * m + 1] << 16) - bias);
-}
+// LUT16T entries v0 .. v0+3 (UPPER: v0, v0+1) of the lane's sixteen channels.
+template <bool UPPER> struct Src { unsigned d[16][UPPER ? 1 : 2]; };
 
-// Table-build registers: the LUT16T dwords (entries v0, v0+1) of the wave's
-// eight channels.
-struct Rows { unsigned d[8]; };
-// Eight weight indices (channels o0 + 8*og .. +7) at k, wcol = &wt[k][o0 +
-// 8*og].  Lane parity picks the dword (indices 0-3 / 4-7) so the load is a
-// vector load: a scalar load would share the LDS wait counter and,
-// completing out of order, force every LDS wait of the step to drain it.
-__device__ __forceinline__ unsigned load_w8(const uint8_t* wcol, int lane) {
-  return __builtin_amdgcn_raw_buffer_load_b32(buffer_rsrc(wcol, 8), (lane & 1) * 4, 0, 0);
-}
-
-// Dword at entries (v0, v0+1) of LUT16T row w_c for every channel c of the
-// group, v0 = 2*lane + sbase/2.  Row offsets are wave-uniform (read from
-// lanes 0 and 1 of the weight-index register).
-__device__ __forceinline__ void load_rows(Rows& r, __amdgpu_buffer_rsrc_t lut, unsigned wv,
-                                          int lane, int sbase) {
-  const unsigned w_lo = __builtin_amdgcn_readlane(wv, 0);
-  const unsigned w_hi = __builtin_amdgcn_readlane(wv, 1);
-#pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    const unsigned wc = ((c < 4 ? w_lo : w_hi) >> (8 * (c & 3))) & 255u;
-    r.d[c] = __builtin_amdgcn_raw_buffer_load_b32(lut, lane * 4, (int)(wc * 512u) + sbase, 0);
-  }
-}
-
-// Writes the lane's two 16-byte chunks (rows v0 and v0+1, channels
-// 8*og .. 8*og+7) at smem + wb (row v0's chunk; row v0+1 is one line on).
-// Signed tables get their even channels' entries biased (LOW_BIAS).
-template <bool SIGNED>
-__device__ __forceinline__ void write_table(unsigned char* smem, const Rows& r, int wb) {
-  unsigned d[8];
-#pragma unroll
-  for (int c = 0; c < 8; ++c)
-    d[c] = (SIGNED && (c & 1) == 0) ? r.d[c] ^ (LOW_BIAS | (LOW_BIAS << 16)) : r.d[c];
-  uint4 lo, hi;      // channel pairs (2m, 2m+1) at v0 (low halves) / v0+1 (high)
-  lo.x = __builtin_amdgcn_perm(d[1], d[0], 0x05040100u);
-  lo.y = __builtin_amdgcn_perm(d[3], d[2], 0x05040100u);
-  lo.z = __builtin_amdgcn_perm(d[5], d[4], 0x05040100u);
-  lo.w = __builtin_amdgcn_perm(d[7], d[6], 0x05040100u);
-  hi.x = __builtin_amdgcn_perm(d[1], d[0], 0x07060302u);
-  hi.y = __builtin_amdgcn_perm(d[3], d[2], 0x07060302u);
-  hi.z = __builtin_amdgcn_perm(d[5], d[4], 0x07060302u);
-  hi.w = __builtin_amdgcn_perm(d[7], d[6], 0x07060302u);
-  *(uint4*)(smem + wb) = lo;
-  *(uint4*)(smem + wb + LINE) = hi;
-}
-
-// Accumulates one table for this lane's RPL rows.  x holds the rows'
-// offsets (two per dword, below 65536); gx XORs in the lane's channel chunk
-// (bits 4-5), the table's quarter (bits 6-7) and the quad buffer (bit 16).
-// All sixteen reads are issued before the first add, so the lane has a whole
-// table step of reads in flight (2.5% faster than two batches of eight).
-template <bool SIGNED>
-__device__ __forceinline__ void use_table(int (&acc)[RPL][8], const unsigned char* smem,
-                                          const XRows& x, unsigned gx) {
-  uint4 e[RPL];
-#pragma unroll
-  for (int h = 0; h < NQ; ++h) {
-    e[RQ * h] = *(const uint4*)(smem + ((x.v[h].x & 0xffffu) ^ gx));
-    e[RQ * h + 1] = *(const uint4*)(smem + ((x.v[h].x >> 16) ^ gx));
-    e[RQ * h + 2] = *(const uint4*)(smem + ((x.v[h].y & 0xffffu) ^ gx));
-    e[RQ * h + 3] = *(const uint4*)(smem + ((x.v[h].y >> 16) ^ gx));
-  }
-#pragma unroll
-  for (int j = 0; j < RPL; ++j) add8<SIGNED>(acc[j], e[j]);
-}
-
-// Stores W consecutive results v[0..W-1] of channel o at y[yi..yi+W-1] as
-// int32 (kind ATX_OUT_I32, also the split-K partials), fp32, or dequantized
-// fp32 (sx * sw[o] * v [+ bias[o]]).
-template <int KIND, int W>
-__device__ __forceinline__ void put_rows(const GemmParams& p, void* y, long long yi,
-                                         int o, const int* v) {
-  if constexpr (KIND == ATX_OUT_I32) {
-    if constexpr (W == 4) *(int4*)((int*)y + yi) = make_int4(v[0], v[1], v[2], v[3]);
-    else ((int*)y)[yi] = v[0];
+// Loads them: w holds the sixteen weight indices; base is v0 in byte 0 and,
+// for a tap past the end, bit 30 (the address then lies past the image and
+// the entries read 0).
+template <bool UPPER>
+__device__ __forceinline__ void load_src(Src<UPPER>& s, int c, __amdgpu_buffer_rsrc_t lut,
+                                         const v4i w, unsigned base) {
+  const unsigned sel = 0x03020000u | (unsigned)(4 + (c & 3)) << 8;
+  const unsigned off = __builtin_amdgcn_perm((unsigned)w[c >> 2], base, sel) << 1;
+  if constexpr (UPPER) {
+    s.d[c][0] = __builtin_amdgcn_raw_buffer_load_b32(lut, (int)off, 0, 0);
   } else {
-    float f[W];
-    if constexpr (KIND == ATX_OUT_F32) {
-#pragma unroll
-      for (int m = 0; m < W; ++m) f[m] = (float)v[m];
-    } else {
-      const float sc = p.sx[0] * p.sw[o];
-#pragma unroll
-      for (int m = 0; m < W; ++m) {
-        const float t = (float)v[m] * sc;
-        f[m] = p.bias ? p.bias[o] + t : t;
-      }
-    }
-    if constexpr (W == 4) *(float4*)((float*)y + yi) = make_float4(f[0], f[1], f[2], f[3]);
-    else ((float*)y)[yi] = f[0];
+    const uint2 v = __builtin_bit_cast(
+        uint2, __builtin_amdgcn_raw_buffer_load_b64(lut, (int)off, 0, 0));
+    s.d[c][0] = v.x;
+    s.d[c][1] = v.y;
   }
 }
 
-// Writes the lane's accumulators: channel o0 + e, rows r + NRG*RQ*h + m of
-// quad h (r = first row of quad 0).  Rows beyond R and channels beyond O are
-// dropped.  With L % 4 == 0 a quad never straddles two images and is one
-// 16-byte store (r is a multiple of 4); otherwise rows are stored one by one,
-// stepping (n, l) across image boundaries.
-template <int KIND>
-__device__ __forceinline__ void store_tile(const GemmParams& p, void* y,
-                                           const int (&acc)[RPL][8], int r, int o0) {
+// Chunks of two table rows (e: v0 + 2u, o: v0 + 2u + 1) in both planes.
+struct Chunks { unsigned e0[4], e1[4], o0[4], o1[4]; };
+
+// Channels 4k .. 4k + 3 of entries u: bytes transposed into the rows' chunks
+// (sel0 / sel1 pick the planes' bytes).
+template <bool UPPER>
+__device__ __forceinline__ void transpose4(Chunks& t, const Src<UPPER>& s, int u, int k,
+                                           unsigned sel0, unsigned sel1, unsigned xk) {
+  const unsigned d0 = s.d[4 * k][u] ^ xk, d1 = s.d[4 * k + 1][u] ^ xk;
+  const unsigned d2 = s.d[4 * k + 2][u] ^ xk, d3 = s.d[4 * k + 3][u] ^ xk;
+  const unsigned p01 = __builtin_amdgcn_perm(d1, d0, 0x05010400u);
+  const unsigned p23 = __builtin_amdgcn_perm(d3, d2, 0x05010400u);
+  const unsigned q01 = __builtin_amdgcn_perm(d1, d0, 0x07030602u);
+  const unsigned q23 = __builtin_amdgcn_perm(d3, d2, 0x07030602u);
+  t.e0[k] = __builtin_amdgcn_perm(p23, p01, sel0);
+  t.e1[k] = __builtin_amdgcn_perm(p23, p01, sel1);
+  t.o0[k] = __builtin_amdgcn_perm(q23, q01, sel0);
+  t.o1[k] = __builtin_amdgcn_perm(q23, q01, sel1);
+}
+
+// Stores the chunks: the lane's first plane at wa, the other at wb.
+__device__ __forceinline__ void store_chunks(unsigned char* smem, const Chunks& t, int u,
+                                             unsigned wa, unsigned wb) {
+  *(uint4*)(smem + wa + (2 * u) * LINE) = make_uint4(t.e0[0], t.e0[1], t.e0[2], t.e0[3]);
+  *(uint4*)(smem + wb + (2 * u) * LINE) = make_uint4(t.e1[0], t.e1[1], t.e1[2], t.e1[3]);
+  *(uint4*)(smem + wa + (2 * u + 1) * LINE) = make_uint4(t.o0[0], t.o0[1], t.o0[2], t.o0[3]);
+  *(uint4*)(smem + wb + (2 * u + 1) * LINE) = make_uint4(t.o1[0], t.o1[1], t.o1[2], t.o1[3]);
+}
+
+// The lane's eight channels of an output tile: index, and for fp32 kinds the
+// factor and bias (ATX_OUT_F32: 1 and none).
+struct OutChannels { int o[8]; float sc[8], b[8]; };
+
+__device__ __forceinline__ OutChannels out_channels(const GemmParams& p, int oc, int lane,
+                                                    bool raw) {
+  OutChannels t;
+  const bool dq = !raw && p.out_kind == ATX_OUT_DEQUANT;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    t.o[e] = oc + 16 * (((lane >> 3) & 1) ^ (e >> 2)) + 4 * (lane >> 4) + (e & 3);
+    const int o = min(t.o[e], p.O - 1);
+    t.sc[e] = dq ? p.sx[0] * p.sw[o] : 1.0f;
+    t.b[e] = dq && p.bias ? p.bias[o] : 0.0f;
+  }
+  return t;
+}
+
+// One output value's bits: the int32 sum (`raw`), or fp32 sc * sum [+ bias].
+__device__ __forceinline__ int out_bits(int v, float sc, float b, bool raw, bool bias) {
+  if (raw) return v;
+  const float t = (float)v * sc;
+  return __builtin_bit_cast(int, bias ? b + t : t);
+}
+
+// Writes the lane's accumulators: rows r + 64 h .. + 3 (r a multiple of 4) of
+// its channels, to y as int32 (`raw`: split-K partials too) or fp32.
+// Rows beyond R and channels beyond O are dropped.  With L % 4 == 0 four rows
+// never straddle two images and are one 16-byte store; otherwise rows are
+// stored one by one, stepping (n, l) across image boundaries.
+__device__ __forceinline__ void store_tile(const GemmParams& p, int* y, const Acc& acc, int r,
+                                           int oc, int lane, bool raw) {
+  const bool bias = !raw && p.out_kind == ATX_OUT_DEQUANT && p.bias;
+  const OutChannels t = out_channels(p, oc, lane, raw);
   const bool vec = (p.L & 3) == 0;
 #pragma unroll
-  for (int h = 0; h < NQ; ++h) {
-    const int rq = r + NRG * RQ * h;
+  for (int h = 0; h < RPL / 4; ++h) {
+    const int rq = r + 64 * h;
     if (rq >= p.R) break;
-    const int n = rq / p.L;
-    const int l = rq - n * p.L;
+    int n = rq / p.L, l = rq - n * p.L;
     if (vec) {
       const long long ybase = (long long)n * p.O * p.L + l;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const int o = o0 + e;
-        if (o >= p.O) break;
-        const int v[RQ] = {acc[RQ * h][e], acc[RQ * h + 1][e], acc[RQ * h + 2][e],
-                           acc[RQ * h + 3][e]};
-        put_rows<KIND, RQ>(p, y, ybase + (long long)o * p.L, o, v);
+        if (t.o[e] >= p.O) continue;
+        int v[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+          v[m] = out_bits(acc[4 * h + m][e >> 2][e & 3], t.sc[e], t.b[e], raw, bias);
+        *(int4*)(y + ybase + (long long)t.o[e] * p.L) = make_int4(v[0], v[1], v[2], v[3]);
       }
     } else {
-      int nm = n, lm = l;
 #pragma unroll
-      for (int m = 0; m < RQ; ++m) {
+      for (int m = 0; m < 4; ++m) {
         if (rq + m >= p.R) break;
-        const long long ybase = (long long)nm * p.O * p.L + lm;
+        const long long ybase = (long long)n * p.O * p.L + l;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int o = o0 + e;
-          if (o >= p.O) break;
-          put_rows<KIND, 1>(p, y, ybase + (long long)o * p.L, o, &acc[RQ * h + m][e]);
-        }
-        if (++lm == p.L) { lm = 0; ++nm; }
+        for (int e = 0; e < 8; ++e)
+          if (t.o[e] < p.O)
+            y[ybase + (long long)t.o[e] * p.L] =
+                out_bits(acc[4 * h + m][e >> 2][e & 3], t.sc[e], t.b[e], raw, bias);
+        if (++l == p.L) { l = 0; ++n; }
       }
     }
   }
 }
 
 // Sums of one tile segment: rows tile tr, channels tile to, k in [kb, ke).
-template <bool SIGNED, bool UPPER>
+template <bool UPPER>
 __device__ __forceinline__ void lut_tile(const GemmParams& p, unsigned char* smem, int tr,
-                                         int to, int kb, int ke, int (&acc)[RPL][8]) {
+                                         int to, int kb, int ke, Acc& acc) {
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
-  const int rg = lane / CG, g = lane % CG;
-  const int o0 = to * OT;
+  const int j16 = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int b = 0; b < RPL; ++b)
+#pragma unroll
+    for (int c = 0; c < 2; ++c) acc[b][c] = v4i{0, 0, 0, 0};
+  if (kb >= ke) return;
 
-  // Table build: wave w writes channel group og = w % 4 for rows
-  // 128 hw .. 128 hw + 127 (hw = w / 4); lane t the row pair v0 = 128 hw + 2t,
-  // v0 + 1, whose chunk og sits at position og ^ ((v0 >> 1) & 3) =
-  // og ^ (t & 3) of quarter q.  wb0 addresses row v0's chunk in quad
-  // buffer 0 (buffer 1 is QTAB on); the quarter is an immediate offset
-  // (q * 64).
-  //
-  // UPPER (every activation index >= 128): tables hold rows 128..255 only.
-  // They are built in pairs, wave w writing rows 128..255 of channel group og
-  // of table 2i + hw: in an even sub-step every wave loads the weight indices
-  // of the next pair and writes its table of the current pair, in an odd one
-  // it loads the LUT rows of the next pair and writes nothing, so each wave
-  // does half the table work of full tables.  Row 0 (the operand's padding
-  // rows and taps point there) is set once per kernel to a zero entry.
-  const int og = __builtin_amdgcn_readfirstlane(wave % CG);
-  const int hw = __builtin_amdgcn_readfirstlane(wave / CG);
-  const int vbase = UPPER ? 128 : 128 * hw;             // first table row of the lane pairs
-  const int tsel = UPPER ? hw : 0;                      // the wave's table of a pair
-  const int sbase = 2 * vbase;                          // its byte offset in a LUT16T row
-  const int wb0 = (vbase + 2 * lane) * LINE + ((og ^ (lane & 3)) << 4);
-  // Read XOR masks: sub-step s of a quad reads quarter (rg + s) & 3.
-  const unsigned gbase = (unsigned)((rg << 6) | (g << 4));
+  // Reads: lane (j, g) reads the tap of quarter t = (j & 3) ^ g, which for its
+  // rows (64 h + 4 j + m) sits in operand slot (t - j) & 3.  t and the channel
+  // half j >> 3 differ between the lanes of a read pass that share a plane.
+  const int tq = (j16 & 3) ^ g;
+  unsigned mask = (unsigned)(tq << 6 | (j16 >> 3) << 5 | (g & 1) << 4);
+  const Select sel = make_select(lane);
 
-  const int xoff = (wave * RPW + rg * RQ) * 2;          // lane's first quad, bytes
+  // Table build: wave w builds table t = w & 3 of the quad for its rows
+  // vh .. vh + 127 (vh = 128 (w >> 2); UPPER: 64 rows of 128..255); lane bit
+  // 1 is the channel half, the other bits the group of four (UPPER: two) rows
+  // v0.  The four lanes of a store pass write four 16-byte positions: two
+  // channel halves, and the planes in the order of lane bit 0.
+  const int bt = wave & 3, bcg = (lane >> 1) & 1, vg = (lane >> 2) << 1 | (lane & 1);
+  const int v0 = UPPER ? 128 + 64 * (wave >> 2) + 2 * vg : 128 * (wave >> 2) + 4 * vg;
+  const unsigned wline = (unsigned)(v0 * LINE + bt * 64 + bcg * 32);
+  unsigned wa = wline + (vg & 1) * 16, wb = wline + (~vg & 1) * 16;
+  const unsigned sel0 = (vg & 1) ? 0x05040100u : 0x07060302u;   // low / high bytes
+  const unsigned sel1 = (vg & 1) ? 0x07060302u : 0x05040100u;
+  const unsigned xk = code_xor(p.sgn);
+  const __amdgpu_buffer_rsrc_t lutr = buffer_rsrc(p.lut16t, 256 * 256 * 2);
+
+  const int n = ke - kb;
+  const int nq = (n + TPL - 1) / TPL;
+  const int slot_bytes = p.Rpad * 2;                    // one k-row of the operand
+  const int xoff = ((tq - j16) & 3) * slot_bytes + (wave * RPW + j16 * 4) * 2;
   const uint16_t* __restrict__ xtile = p.xt + (long long)tr * p.rt;
   // wave-uniform: does this wave own rows of the tile?
   const bool active = __builtin_amdgcn_readfirstlane(wave) * RPW < p.rt;
-  const uint8_t* __restrict__ wcol = p.wt + o0 + og * 8;
-  const __amdgpu_buffer_rsrc_t lutr = buffer_rsrc(p.lut16t, 256 * 256 * 2);
-  // Zero-length view of the image: its loads are out of range and return 0,
-  // which builds an all-zero table for the steps past the chunk's end.
-  const __amdgpu_buffer_rsrc_t lutz = buffer_rsrc(p.lut16t, 0);
+  // Quads past the chunk read through an empty view (0); a wave past the tile,
+  // whose rows can lie past the operand's padded rows when a short last tile
+  // ends near Rpad, reads none.
+  auto load_x = [&](int j, int h) {                     // rows 64 h + 4 j16 .. + 3
+    // (readfirstlane: a select, not a branch)
+    const int bytes = __builtin_amdgcn_readfirstlane(j < nq ? TPL * slot_bytes : 0);
+    const __amdgpu_buffer_rsrc_t xs =
+        buffer_rsrc(xtile + (long long)(kb + TPL * j) * p.Rpad, bytes);
+    return __builtin_bit_cast(
+        uint2, __builtin_amdgcn_raw_buffer_load_b64(xs, xoff, 128 * h, 0));
+  };
+  // The lane's sixteen weight indices of quad j (0 past the chunk).
+  const uint8_t* __restrict__ wtile = p.wt + to * OT;
+  const int woff = bt * p.Opad + bcg * 16;
+  auto load_w = [&](int j) {
+    const int taps = min(TPL, n - TPL * j);
+    const __amdgpu_buffer_rsrc_t ws =
+        buffer_rsrc(wtile + (long long)(kb + TPL * min(j, nq - 1)) * p.Opad,
+                    taps > 0 ? (taps - 1) * p.Opad + OT : 0);
+    return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(ws, woff, 0, 0));
+  };
+  auto src_base = [&](int j) {
+    return (unsigned)v0 | (TPL * j + bt < n ? 0u : 0x40000000u);
+  };
 
+  Src<UPPER> src;
+  v4i wreg;
+  constexpr int NU = UPPER ? 1 : 2;                     // row pairs a lane builds
+  Chunks t;
+  // Part i of a table build: channels 4k .. 4k + 3 of row pair u.
+  auto piece = [&](int i) __attribute__((always_inline)) {
+    const int u = i / 4, k = i % 4;
+    transpose4<UPPER>(t, src, u, k, sel0, sel1, xk);
+    if (k == 3) store_chunks(smem, t, u, wa, wb);
+  };
+  auto load_all = [&](const v4i w, int j) __attribute__((always_inline)) {
 #pragma unroll
-  for (int j = 0; j < RPL; ++j)
+    for (int c = 0; c < 16; ++c) load_src<UPPER>(src, c, lutr, w, src_base(j));
+  };
+  wreg = load_w(1);
+  load_all(load_w(0), 0);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc[j][e] = 0;
+  for (int i = 0; i < 4 * NU; ++i) piece(i);            // quad 0 -> buffer 0
+  load_all(wreg, 1);
 
-  if (kb < ke) {
-    // Sub-steps sigma = 4j + s (tables counted from kb; n of them).  Sub-step
-    // sigma issues the loads for the row offsets of sub-step sigma+1, the
-    // LUT rows of table sigma+5 and the weight indices of table sigma+6,
-    // accumulates from the lane's table of sub-step sigma and writes table
-    // sigma+4 (rows loaded one sub-step earlier).  Tables at or past n are
-    // built all-zero from lutz; row offsets past the chunk load as 0 (row 0
-    // of such a table), so whole quads run without branches.  Scheduling
-    // fences keep the loads ahead of the accumulation and the table write
-    // (which waits for its LUT rows) behind it.
-    const int n = ke - kb;
-    const int nq = (n + TPL - 1) / TPL;
-    const int slot_bytes = p.Rpad * 2;                  // one k-row of the operand
-    // The operand's quads are rotated (slot s of row r holds tap
-    // 4j + (((r >> 2) + s) & 3)), so at sub-step s every lane reads slot s:
-    // a scalar offset.  Quads past the chunk, and every quad of a wave past
-    // the tile (whose rows can lie past the operand's padded rows when a
-    // short last tile ends near Rpad), read through an empty view (0).
-    auto quad_rows = [&](int j) {                       // descriptor of quad j's slots
-      return buffer_rsrc(xtile + (long long)(kb + TPL * j) * p.Rpad,
-                         j < nq && active ? TPL * slot_bytes : 0);
-    };
-    auto wtab = [&](int t) {                            // weight column of table t
-      return wcol + (long long)(kb + min(t, n - 1)) * p.Opad;
-    };
-
-    XRows xa, xb;
-    Rows rows;
-    unsigned wnext = 0;                                 // indices of table sigma+5 (UPPER:
-                                                        // of the wave's table of the next pair)
-    {
-      Rows r4;
-      if constexpr (UPPER) {
-#pragma unroll
-        for (int q = 0; q < TPL; q += 2) {
-          load_rows(r4, q + tsel < n ? lutr : lutz, load_w8(wtab(q + tsel), lane), lane, sbase);
-          write_table<SIGNED>(smem + (q + tsel) * 64, r4, wb0);  // quad 0 -> buffer 0
-        }
-      } else {
-#pragma unroll
-        for (int q = 0; q < TPL; ++q) {
-          load_rows(r4, q < n ? lutr : lutz, load_w8(wtab(q), lane), lane, sbase);
-          write_table<SIGNED>(smem + q * 64, r4, wb0);  // quad 0 -> buffer 0
-        }
-      }
-      load_rows(rows, TPL + tsel < n ? lutr : lutz, load_w8(wtab(TPL + tsel), lane), lane,
-                sbase);
-      if constexpr (!UPPER) wnext = load_w8(wtab(TPL + 1), lane);
-      load_x(xa, quad_rows(0), xoff, 0);
-    }
+  if (!active) {                                        // tables only
     __syncthreads();
-
-    // One sub-step; B = quad buffer of quad j, S = sub-step within the quad.
-    auto sub = [&](auto bc, auto sc, int j, XRows& xcur, XRows& xnext)
-        __attribute__((always_inline)) {
-      constexpr int B = decltype(bc)::value;
-      constexpr int S = decltype(sc)::value;
-      const int sigma = TPL * j + S;
-      // Issue order = order of use in the next sub-step (the counter of
-      // outstanding loads is waited on in order): weight indices (first, to
-      // address the LUT rows), row offsets (the accumulation), LUT rows
-      // (the table write at the end).  UPPER: even sub-steps load the
-      // indices of the pair (sigma+6, sigma+7) and write table sigma+4+hw,
-      // odd ones load the LUT rows of table sigma+5+hw.
-      constexpr bool kIdx = !UPPER || (S & 1) == 0;     // loads weight indices
-      constexpr bool kRows = !UPPER || (S & 1) == 1;    // loads LUT rows
-      unsigned wn = wnext;
-      if constexpr (kIdx) wn = load_w8(wtab(sigma + 6 + tsel), lane);
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (S + 1 < TPL) load_x(xnext, quad_rows(j), xoff, (S + 1) * slot_bytes);
-      else load_x(xnext, quad_rows(j + 1), xoff, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      Rows rn;
-      if constexpr (kRows)
-        load_rows(rn, sigma + 5 + tsel < n ? lutr : lutz, wnext, lane, sbase);
-      __builtin_amdgcn_sched_barrier(0);
-      if (active) {
-        use_table<SIGNED>(acc, smem, xcur, quarter_mask<S, B>(gbase));
-        // Pin the adds here: left free, the compiler sinks them into later
-        // steps, past the table write that waits for this step's loads.
+    for (int j = 0; j < nq; ++j) {
+      wreg = load_w(j + 2);
+      wa ^= QTAB;
+      wb ^= QTAB;
 #pragma unroll
-        for (int jj = 0; jj < RPL; ++jj)
-#pragma unroll
-          for (int e = 0; e < 8; ++e) asm volatile("" : "+v"(acc[jj][e]));
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      if constexpr (kIdx)                               // table sigma+4 (+hw), other buffer
-        write_table<SIGNED>(smem + (S + tsel) * 64 + (B ? 0 : QTAB), rows, wb0);
-      if constexpr (kRows) rows = rn;
-      wnext = wn;
-      if constexpr (S == TPL - 1) __syncthreads();
-    };
-    using I0 = std::integral_constant<int, 0>;
-    using I1 = std::integral_constant<int, 1>;
-    using I2 = std::integral_constant<int, 2>;
-    using I3 = std::integral_constant<int, 3>;
-    for (int j = 0; j < nq; j += 2) {
-      sub(I0{}, I0{}, j, xa, xb);
-      sub(I0{}, I1{}, j, xb, xa);
-      sub(I0{}, I2{}, j, xa, xb);
-      sub(I0{}, I3{}, j, xb, xa);
-      if (j + 1 >= nq) break;
-      sub(I1{}, I0{}, j + 1, xa, xb);
-      sub(I1{}, I1{}, j + 1, xb, xa);
-      sub(I1{}, I2{}, j + 1, xa, xb);
-      sub(I1{}, I3{}, j + 1, xb, xa);
+      for (int i = 0; i < 4 * NU; ++i) piece(i);
+      load_all(wreg, j + 2);
+      __syncthreads();
     }
-    pair_sums<SIGNED>(acc, TPL * nq);
+    return;
   }
+
+  uint2 x[4];                                           // row offsets
+#pragma unroll
+  for (int h = 0; h < 4; ++h) x[h] = load_x(0, h);
+  __syncthreads();
+  for (int j = 0; j < nq; ++j) {
+    // Table of quad j + 1: its entries were loaded during the previous quad;
+    // the entry loads of quad j + 2 follow once the registers are free, one
+    // channel per read pair, so neither the address unit's queue nor the
+    // stores' waits stall the reads.
+    wreg = load_w(j + 2);
+    const unsigned base = src_base(j + 2);
+    wa ^= QTAB;
+    wb ^= QTAB;
+    v8i ring[RD];
+    auto read = [&](int i) __attribute__((always_inline)) {
+      const int b = i >> 1, c = i & 1;
+      const unsigned xd = (b & 2) ? x[b >> 2].y : x[b >> 2].x;
+      const unsigned a = __builtin_amdgcn_perm(xd, mask, (b & 1) ? 0x03020700u : 0x03020500u) ^
+                         (c << 5);
+      const v4i lo = *(const v4i*)(smem + a);
+      const v4i hi = *(const v4i*)(smem + (a ^ 16));
+      ring[i % RD] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+    auto sum = [&](int i, const v4i w) __attribute__((always_inline)) {
+      v4i& a = acc[i >> 1][i & 1];
+      a = __builtin_amdgcn_smfmac_i32_16x16x128_i8(w, ring[i % RD], a, sel.idx, 0, 0);
+    };
+#pragma unroll
+    for (int i = 0; i < RD; ++i) read(i);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 2 * RPL; i += 2) {              // row block i / 2
+      sum(i, sel.both);
+      sum(i + 1, sel.both);
+      sum(i, sel.high);
+      if (i + RD < 2 * RPL) read(i + RD);
+      sum(i + 1, sel.high);
+      if (i + 1 + RD < 2 * RPL) read(i + 1 + RD);
+      if (i / 2 < 4 * NU) piece(i / 2);
+      if (i >= 16) {
+        load_src<UPPER>(src, i - 16, lutr, wreg, base);
+        load_src<UPPER>(src, i - 15, lutr, wreg, base);
+      }
+      if ((i + RD) % 8 == 0 && i + RD < 2 * RPL + 8)    // a row quad has been read
+        x[(i + RD) / 8 - 1] = load_x(j + 1, (i + RD) / 8 - 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    mask ^= QTAB;
+    __syncthreads();
+  }
+  const int total = code_bias(p.sgn) * (TPL * nq);      // mod 2^32, as the sums
+#pragma unroll
+  for (int b = 0; b < RPL; ++b)
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc[b][c][q] = (int)((unsigned)total - (unsigned)acc[b][c][q]);
 }
 
 // Slot layout of a cut tile (stream-K): value (h, m, e) of thread tid at
@@ -695,92 +689,77 @@ __device__ __forceinline__ int sk_slot_tile(const GemmParams& p, int b, long lon
   return (t * p.nqt) / p.sk_per == b ? (int)t : -1;
 }
 
-template <bool SIGNED>
 __global__ void __launch_bounds__(NT, 1)
 lut_gemm_kernel(const GemmParams p) {
   __shared__ __align__(16) unsigned char smem[SMEM_BYTES];
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
-  const int rg = lane / CG, g = lane % CG;
   const int lb = logical_block();
-  int acc[RPL][8];
-  const bool has_rows = wave * RPW < p.rt;   // the wave's rows lie in the tile
+  Acc acc;
+  // the wave's rows lie in the tile
+  const bool has_rows = __builtin_amdgcn_readfirstlane(wave) * RPW < p.rt;
+  const int rlane = wave * RPW + (lane & 15) * 4;       // the lane's first row in the tile
   const bool upper = p.x_upper && __builtin_amdgcn_readfirstlane(*p.x_upper) != 0;
   if (upper && tid < 2 * (LINE / 16)) {      // row 0 (line 0) of both quad buffers
-    // a zero entry as the table build stores it: signed tables hold their
-    // even channels biased by LOW_BIAS, which pair_sums takes off per table
-    const unsigned z = SIGNED ? LOW_BIAS : 0u;
+    // a zero entry as the table build codes it (planes alternate)
+    const unsigned xk = code_xor(p.sgn);
+    const unsigned z = (tid & 1) ? 0x80808080u : (xk >> 24) * 0x01010101u;
     const int c = tid % (LINE / 16);
     *(uint4*)(smem + (tid < LINE / 16 ? 0 : QTAB) + 16 * c) = make_uint4(z, z, z, z);
   }
-
-  if (p.sk_per == 0) {
-    int l = lb;
-    const int to = l % p.tiles_o; l /= p.tiles_o;
-    const int tr = l % p.tiles_r;
-    const int s = l / p.tiles_r;
-    const int kb = s * p.k_chunk;
-    if (upper) lut_tile<SIGNED, true>(p, smem, tr, to, kb, min(p.K, kb + p.k_chunk), acc);
-    else lut_tile<SIGNED, false>(p, smem, tr, to, kb, min(p.K, kb + p.k_chunk), acc);
-    // ---- epilogue: registers -> HBM, every wave at once (no LDS staging).
-    const int r0 = tr * p.rt + wave * RPW + rg * RQ;     // this lane's first quad
-    const int oc = to * OT + g * 8;
-    if (!has_rows) return;
-    if (p.splits > 1)
-      store_tile<ATX_OUT_I32>(p, (int*)p.y + (long long)s * p.split_stride, acc, r0, oc);
-    else if (p.out_kind == ATX_OUT_I32)
-      store_tile<ATX_OUT_I32>(p, p.y, acc, r0, oc);
-    else if (p.out_kind == ATX_OUT_F32)
-      store_tile<ATX_OUT_F32>(p, p.y, acc, r0, oc);
-    else
-      store_tile<ATX_OUT_DEQUANT>(p, p.y, acc, r0, oc);
-    return;
-  }
-
-  // Whole tiles first (the full rounds), then this workgroup's run of the
-  // remaining tiles' quads, tile segment by tile segment.
-  for (int tile = lb; tile < p.sk_dp; tile += p.sk_g) {
-    const int to = tile % p.tiles_o, tr = tile / p.tiles_o;
-    __syncthreads();                         // the previous segment's tables are read
-    if (upper) lut_tile<SIGNED, true>(p, smem, tr, to, 0, p.K, acc);
-    else lut_tile<SIGNED, false>(p, smem, tr, to, 0, p.K, acc);
-    const int r0 = tr * p.rt + wave * RPW + rg * RQ;
-    const int oc = to * OT + g * 8;
-    if (!has_rows) continue;
-    if (p.out_kind == ATX_OUT_I32) store_tile<ATX_OUT_I32>(p, p.y, acc, r0, oc);
-    else if (p.out_kind == ATX_OUT_F32) store_tile<ATX_OUT_F32>(p, p.y, acc, r0, oc);
-    else store_tile<ATX_OUT_DEQUANT>(p, p.y, acc, r0, oc);
-  }
+  // Segments: one tile's k-chunk (split-K), or (stream-K) whole tiles first
+  // (the full rounds), then this workgroup's run of the remaining tiles'
+  // quads, tile segment by tile segment.
   const long long total = ((long long)p.tiles_r * p.tiles_o - p.sk_dp) * p.nqt;
   long long it = (long long)lb * p.sk_per;
   const long long end = min(total, it + p.sk_per);
-  while (it < end) {
-    const int tt = (int)(it / p.nqt);        // tail tile
-    const int q0 = (int)(it - (long long)tt * p.nqt);
-    const int q1 = (int)min((long long)p.nqt, q0 + (end - it));
-    const int tile = p.sk_dp + tt;
-    const int to = tile % p.tiles_o, tr = tile / p.tiles_o;
-    __syncthreads();                         // the previous segment's tables are read
-    if (upper) lut_tile<SIGNED, true>(p, smem, tr, to, TPL * q0, min(p.K, TPL * q1), acc);
-    else lut_tile<SIGNED, false>(p, smem, tr, to, TPL * q0, min(p.K, TPL * q1), acc);
-    if (!has_rows) {
-      // nothing to store or add (the slots' rows of this wave stay zero)
-    } else if (q0 == 0 && q1 == p.nqt) {
-      const int r0 = tr * p.rt + wave * RPW + rg * RQ;
-      const int oc = to * OT + g * 8;
-      if (p.out_kind == ATX_OUT_I32) store_tile<ATX_OUT_I32>(p, p.y, acc, r0, oc);
-      else if (p.out_kind == ATX_OUT_F32) store_tile<ATX_OUT_F32>(p, p.y, acc, r0, oc);
-      else store_tile<ATX_OUT_DEQUANT>(p, p.y, acc, r0, oc);
+  int whole = p.sk_per ? lb : p.sk_dp;                   // next whole tile
+  for (bool first = true;; first = false) {
+    int tile, kb, ke;
+    int* slot = nullptr;
+    int* y = (int*)p.y;
+    if (p.sk_per == 0) {
+      if (!first) break;
+      const int nt = p.tiles_o * p.tiles_r, s = lb / nt;
+      tile = lb - s * nt;
+      kb = s * p.k_chunk;
+      ke = min(p.K, kb + p.k_chunk);
+      if (p.splits > 1) y += (long long)s * p.split_stride;
+    } else if (whole < p.sk_dp) {
+      tile = whole;
+      whole += p.sk_g;
+      kb = 0;
+      ke = p.K;
+    } else if (it < end) {
+      const int tt = (int)(it / p.nqt);                  // tail tile
+      const int q0 = (int)(it - (long long)tt * p.nqt);
+      const int q1 = (int)min((long long)p.nqt, q0 + (end - it));
+      tile = p.sk_dp + tt;
+      kb = TPL * q0;
+      ke = min(p.K, TPL * q1);
+      if (q0 != 0 || q1 != p.nqt)
+        slot = p.skws + (((long long)tt * p.nqt) / p.sk_per) * (long long)(RPL * 8 * NT);
+      it += q1 - q0;
     } else {
-      int* slot = p.skws + (((long long)tt * p.nqt) / p.sk_per) * (long long)(RPL * 8 * NT);
+      break;
+    }
+    const int to = tile % p.tiles_o, tr = tile / p.tiles_o;
+    if (!first) __syncthreads();             // the previous segment's tables are read
+    if (upper) lut_tile<true>(p, smem, tr, to, kb, ke, acc);
+    else lut_tile<false>(p, smem, tr, to, kb, ke, acc);
+    // ---- epilogue: registers -> HBM, every wave at once (no LDS staging).
+    if (!has_rows) continue;                 // (a slot's rows of this wave stay zero)
+    if (slot) {
 #pragma unroll
-      for (int j = 0; j < RPL; ++j)
+      for (int b = 0; b < RPL; ++b)
 #pragma unroll
         for (int e = 0; e < 8; ++e)
-          __hip_atomic_fetch_add(slot + sk_index(j, e, tid), acc[j][e], __ATOMIC_RELAXED,
-                                 __HIP_MEMORY_SCOPE_AGENT);
+          __hip_atomic_fetch_add(slot + sk_index(b, e, tid), acc[b][e >> 2][e & 3],
+                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else {
+      store_tile(p, y, acc, tr * p.rt + rlane, to * OT, lane,
+                 p.splits > 1 || p.out_kind == ATX_OUT_I32);
     }
-    it += q1 - q0;
   }
 }
 
@@ -803,20 +782,16 @@ sk_finish_kernel(const GemmParams p) {
   const int tile = p.sk_dp + tt;
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
-  const int rg = lane / CG, g = lane % CG;
   const int* slot = p.skws + (long long)blockIdx.x * (RPL * 8 * NT);
-  int acc[RPL][8];
+  Acc acc;
 #pragma unroll
-  for (int j = 0; j < RPL; ++j)
+  for (int b = 0; b < RPL; ++b)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc[j][e] = slot[sk_index(j, e, tid)];
+    for (int e = 0; e < 8; ++e) acc[b][e >> 2][e & 3] = slot[sk_index(b, e, tid)];
   const int to = tile % p.tiles_o, tr = tile / p.tiles_o;
-  const int r0 = tr * p.rt + wave * RPW + rg * RQ;
-  const int oc = to * OT + g * 8;
   if (wave * RPW >= p.rt) return;            // rows past the tile
-  if (p.out_kind == ATX_OUT_I32) store_tile<ATX_OUT_I32>(p, p.y, acc, r0, oc);
-  else if (p.out_kind == ATX_OUT_F32) store_tile<ATX_OUT_F32>(p, p.y, acc, r0, oc);
-  else store_tile<ATX_OUT_DEQUANT>(p, p.y, acc, r0, oc);
+  store_tile(p, (int*)p.y, acc, tr * p.rt + wave * RPW + (lane & 15) * 4, to * OT, lane,
+             p.out_kind == ATX_OUT_I32);
 }
 
 // Split-K reduction: exact int64 sum of int32 partials, then the epilogue.
@@ -1235,6 +1210,7 @@ static int lut_gemm_run(const uint16_t* xt, int Rpad, const uint8_t* wt, int Opa
   p.out_kind = ep.out_kind; p.y = y;
   p.sx = ep.scale_x; p.sw = ep.scale_w; p.bias = ep.bias;
   p.x_upper = ep.x_upper;
+  p.sgn = lut_class == ATX_LUT_I16;
 
   if (lut_class == ATX_LUT_F32) {
     ATX_REQUIRE(lutf32t, "atx_lut_gemm: fp32 class needs the fp32 image");
@@ -1275,10 +1251,7 @@ static int lut_gemm_run(const uint16_t* xt, int Rpad, const uint8_t* wt, int Opa
     }
     int rc = timing_mark(false, stream);
     if (rc != ATX_OK) return rc;
-    if (lut_class == ATX_LUT_I16)
-      hipLaunchKernelGGL(lut_gemm_kernel<true>, dim3(G), dim3(NT), 0, stream, p);
-    else
-      hipLaunchKernelGGL(lut_gemm_kernel<false>, dim3(G), dim3(NT), 0, stream, p);
+    hipLaunchKernelGGL(lut_gemm_kernel, dim3(G), dim3(NT), 0, stream, p);
     rc = check_launch("lut_gemm_kernel");
     if (rc == ATX_OK) rc = timing_mark(true, stream);
     if (rc != ATX_OK || Gt <= 1) return rc;
@@ -1295,12 +1268,7 @@ static int lut_gemm_run(const uint16_t* xt, int Rpad, const uint8_t* wt, int Opa
   ATX_REQUIRE(blocks < 0x7fffffffLL, "atx_lut_gemm: grid too large");
   int rc = timing_mark(false, stream);
   if (rc != ATX_OK) return rc;
-  if (lut_class == ATX_LUT_I16)
-    hipLaunchKernelGGL(lut_gemm_kernel<true>, dim3((unsigned)blocks), dim3(NT), 0,
-                       stream, p);
-  else
-    hipLaunchKernelGGL(lut_gemm_kernel<false>, dim3((unsigned)blocks), dim3(NT), 0,
-                       stream, p);
+  hipLaunchKernelGGL(lut_gemm_kernel, dim3((unsigned)blocks), dim3(NT), 0, stream, p);
   rc = check_launch("lut_gemm_kernel");
   if (rc == ATX_OK) rc = timing_mark(true, stream);
   if (rc != ATX_OK || pl.splits == 1) return rc;
