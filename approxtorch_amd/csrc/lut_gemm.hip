@@ -881,36 +881,33 @@ struct Plan { int tiles_r, tiles_o, splits, k_chunk, sk_per, nqt, sk_dp, rt; };
 // device query, so the workspace query and the launch always agree.
 constexpr int PLAN_CUS = 256;
 
-// Plan by a cost model in units of one k-step of one full-tile workgroup,
-// over the rows per tile rt (2048, 1792, 1536, 1280 or 768, keeping
-// ceil(R / rt) tiles inside the operand's padded rows) and the split-K count S:
-//   ceil(tiles(rt) * S / CUs) rounds x (k-chunk + 6 fixed steps) x f(rt)
-//   + for S > 1: 4 steps for the reduce launch and S x (R*O / 600000) steps
-//     for writing and re-reading one int32 partial slice,
-// with f(rt) = 0.7 + 0.3 rt / 2048 the cost of a k-step of a smaller tile (the
-// table build, its loads and the quad barrier do not shrink with the rows).
-// Fitted to a sweep of (rt, S) over the 19 distinct ResNet-50 layer shapes
-// at batch 64 (the model's picks land within 0.2% of the sweep's best);
-// rt = 1024 is left out (slower than 768 or 1280 on every shape measured).
+// Plan by a cost model in microseconds, over the rows per tile rt (2048, 1792,
+// 1536, 1280, 1024, 768 or 512, keeping ceil(R / rt) tiles inside the operand's
+// padded rows) and the split-K count S, with x = rt / 2048:
+//   ceil(tiles(rt) * S / CUs) rounds x (k-chunk x step x (0.75 + 0.25 x)
+//     + 3.7 + 5.9 x: table prologue and output stores)
+//   + for S > 1: 3.6 for the reduce launch and S x R*O x 1.31e-6 for writing
+//     and re-reading one int32 partial slice,
+// step = 0.62 (a k-step of a full tile), 0.44 with the upper-half tables
+// (x_upper given: `upper`; the tables' loads and stores halve).  A least-squares
+// fit to a sweep of (rt, S) over 38 shapes (19 ResNet-50 layers at batch 64, 10
+// ResNet-18 layers at 128, GEMM and small shapes), both table heights: its
+// picks take 13.29 ms over the sweep, the best pair of each shape 13.24, the
+// model fitted to the kernel's earlier sums (0.95 us a step) 13.62.
 // k-chunks are whole quads of tables (multiples of 4); S is at least
 // ceil(K / kmax), the exact-int32 bound of one pass, and the smallest cost
 // wins (ties: the larger rt, then the smaller S).
 // Stream-K (K <= kmax, at the default rt): floor(tiles / CUs) full rounds of
 // whole tiles, then the T = tail tiles * ceil(K/4) quads of the rest dealt
 // out evenly, per = ceil(T / CUs) quads per workgroup, which ends the
-// partial last round.  Cost, fitted to the split-K / stream-K times of the
-// 19 distinct ResNet-50 layer shapes at batch 64 (~0.95 us per k-step):
-//   rounds * (K + 14) + 4 * per + 14 per tail segment a workgroup runs
-//   (ceil(per / nqt) + 1 at most; table prologue and atomic sums) + 0.1 per
-//   cut tile (its 256 KiB slot) + 45 for the clear / finish launches.
-// It is taken when cheaper than the best split-K plan (5 of the 19 shapes,
-// e.g. K = 576 at 56 x 56 with 64 channels: 460 against 491 us).  With the
-// upper-half tables (x_upper given: `upper`) a k-step costs ~0.74 us instead
-// of ~0.95 while the cuts' atomics, clears and finishes do not shrink; refit
-// on the four stream-K shapes of the 52 ResNet-50 layers at batch 64, a cut
-// costs ~0.7 k-steps there (0.1 with full tables), which hands K = 576 at
-// 56 x 56 with 64 channels (513 -> 467 us) and K = 512 at 28 x 28 with 256
-// (461 -> 420 us) to split-K.
+// partial last round.  Cost, fitted to the same sweep: the rounds and quads at
+// the step above, a tile's fixed cost per tail segment a workgroup runs
+// (ceil(per / nqt) + 1 at most), 42 for the clear / finish launches and their
+// traffic, 0.07 per cut tile (its 256 KiB slot and atomics).  It is taken when
+// cheaper than the best split-K plan: 5 of the 38 with full tables (K = 1024,
+// 12544 x 512: 327 against 340 us; K = 2304, 12544 x 256: 361 against 370).
+// The upper-half tables' constant is 60: with the slots cold, as within a
+// network, stream-K took 15 us more than split-K at K = 1152, 50176 x 128.
 // ATX_LUT_SCHEDULE (environment: auto | split | stream_k) overrides the
 // choice; ATX_LUT_ROWS and ATX_LUT_SPLITS force the rows per tile and the
 // split count (split-K plans), for measurement.
@@ -938,10 +935,13 @@ static Plan make_plan(int N, int K, int L, int O, int kmax, long long ws_limit =
   const long long cus = PLAN_CUS;
   const int smin = (int)cdiv(K, kmax);
   const int fs = force_s ? std::max(smin, atoi(force_s)) : 0;
-  const double slice = (double)R * O / 600000.0;
+  const double step = upper ? 0.437 : 0.623;               // us per k-step of a full tile
+  const double slice = (double)R * O * 1.31e-6;
+  const auto step_cost = [&](int rt) { return step * (0.753 + 0.247 * rt / RT); };
+  const auto tile_cost = [&](int rt) { return 3.66 + 5.93 * rt / RT; };
   const long long rows_cap = cdiv(R, RT) * RT;
-  static const int kRows[] = {2048, 1792, 1536, 1280, 768};
-  int cand[6], nc = 0;
+  static const int kRows[] = {2048, 1792, 1536, 1280, 1024, 768, 512};
+  int cand[8], nc = 0;
   if (force_rows) {
     const int rt = atoi(force_rows);
     if (rt >= RPW && rt <= RT && rt % RPW == 0 && R > 0 && cdiv(R, rt) * rt <= rows_cap)
@@ -963,14 +963,18 @@ static Plan make_plan(int N, int K, int L, int O, int kmax, long long ws_limit =
   for (int c = 0; c < nc; ++c) {
     const int rt = cand[c];
     const long long tiles = cdiv(R, rt) * pl.tiles_o;
-    const double f = 0.7 + 0.3 * rt / RT;
+    // least cost of S or more splits (no workgroup idle): ends the search early
+    const double work = tiles * (K * step_cost(rt)) / cus;
+    const double per_s = tiles * tile_cost(rt) / cus + slice;
     for (int S = fs ? fs : smin; S <= (fs ? fs : std::max(smin, 64)); ++S) {
       const long long kc = cdiv(cdiv(K, S), TPL) * TPL;
-      if (S > smin && kc < 16 && !fs) break;
+      if (S > smin && kc < 8 && !fs) break;
+      if (found && S > 1 && work + S * per_s >= best_cost) break;
       const long long splits = cdiv(K, kc);
       if (ws_limit >= 0 && splits > 1 && splits * R * O * 4 > ws_limit) continue;
-      const double cost = (double)cdiv(tiles * splits, cus) * (double)(kc + 6) * f +
-                          (splits > 1 ? 4.0 + splits * slice : 0.0);
+      const double cost = (double)cdiv(tiles * splits, cus) *
+                              (kc * step_cost(rt) + tile_cost(rt)) +
+                          (splits > 1 ? 3.6 + splits * slice : 0.0);
       if (!found || cost < best_cost) {
         best_kc = kc; best_cost = cost; best_rt = rt; found = true;
       }
@@ -989,9 +993,10 @@ static Plan make_plan(int N, int K, int L, int O, int kmax, long long ws_limit =
     const long long per = cdiv(T, cus);
     if (per >= 2) {
       const long long cuts = std::min<long long>(tail, cdiv(T, per) - 1);
-      const double sk_cost = (double)rounds * (K + 14) + 4.0 * per +
-                             14.0 * (double)(cdiv(per, pl.nqt) + 1) +
-                             (upper ? 0.7 : 0.1) * cuts + 45.0;
+      const double sk_cost = rounds * (K * step_cost(pl.rt) + tile_cost(pl.rt)) +
+                             4.0 * per * step_cost(pl.rt) +
+                             tile_cost(pl.rt) * (double)(cdiv(per, pl.nqt) + 1) +
+                             (upper ? 60.0 : 42.0) + 0.07 * cuts;
       if (force_sk || sk_cost < best_cost) {
         pl.sk_per = (int)per;
         pl.sk_dp = (int)(rounds * cus);
