@@ -196,7 +196,12 @@ def ptr(t):
 
 
 def stream_of(t):
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """Handle of the current stream of t's device (a raw query: 0.3 us, where
+    torch.cuda.current_stream builds a Stream object in 5 us; a layer's pass
+    asks four to twelve times)."""
+    if t.is_cuda:
+        return torch._C._cuda_getCurrentRawStream(t.get_device())
+    return torch.cuda.current_stream(t.device).cuda_stream    # raises: not a GPU tensor
 
 
 def geom(N, C, H, W, KH, KW, SH, SW, PH, PW, DH, DW):

@@ -4,6 +4,7 @@ same constructor, buffers (lut, scale_x, scale_w, dx, dw), EMA rules and
 forward composition; the per-step statistics, fake-quant and LUT conv run as
 HIP kernels.
 """
+import ctypes
 import math
 
 import torch
@@ -41,7 +42,10 @@ def _bump(*buffers):
 
 def _ema_coeffs(m):
     # torch evaluates `m * cur + (1 - m) * old` with both python scalars cast
-    # to fp32: reproduce those two constants exactly.
+    # to fp32: reproduce those two constants exactly (a Python number is rounded
+    # by ctypes, 0.5 us; a tensor of it costs 5).
+    if type(m) in (float, int):
+        return ctypes.c_float(m).value, ctypes.c_float(1 - m).value
     return float(torch.tensor(m, dtype=torch.float32)), \
         float(torch.tensor(1 - m, dtype=torch.float32))
 
