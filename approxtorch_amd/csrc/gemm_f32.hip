@@ -15,9 +15,10 @@
 // - split-bf16 (the layer paths): fp32 operands split exactly into three
 //   bf16 parts and multiplied on v_mfma_f32_16x16x32_bf16 as the six part
 //   products of order <= 2 (three when a table is bf16 already); see the
-//   "split-bf16 operand planes" section below.  Backward-weight, the
-//   backward-data GEMM of atx_conv_bwd_data (its A operand from bf16 weight
-//   planes prepared per call) and the implicit backward-data GEMM.
+//   "split-bf16 operand planes" section below.  Backward-weight, and for
+//   atx_conv_bwd_data the column GEMM (its A operand from bf16 weight planes
+//   prepared per call) and the tap GEMM (both operands from planes, the image
+//   gradient without columns).
 // - fp32 (v_mfma_f32_16x16x4f32, plain fp32 products): the backward-data
 //   GEMM of atx_conv_bwd_data_col (no workspace for the planes) and layers
 //   whose go spans exceed the split path's 32-bit buffer offsets.  The
@@ -295,124 +296,6 @@ template <int B, bool VEC, bool SCALED> struct DataB {
 // (out-of-range go positions contribute 0).  With O % BK == 0 every k-tile
 // has one tap t, so its spatial shift is uniform over the tile.
 
-// A(m = c, p) = tx[wq[o*K + c*KK + t]], KMajor (quads of four channels).
-template <int B> struct DgradA {
-  using Lay = KMajor<B>;
-  static constexpr int QPR = B / 4, NQ = BK * B / (4 * GT), PSTEP = GT / QPR;
-  const uint8_t* wq; int K, KK, C, O;
-  int mq, pr, gm;
-  unsigned raw[NQ], ok;
-  __device__ void init(int t, int m0) { mq = (t % QPR) * 4; pr = t / QPR; gm = m0 + mq; }
-  __device__ void fetch(int p0, int pe) {
-    const int tap = p0 / O;                   // uniform over the k-tile
-    const int o0 = p0 - tap * O;
-    ok = 0;
-#pragma unroll
-    for (int i = 0; i < NQ; ++i) {
-      const int o = o0 + pr + i * PSTEP;
-      const bool pv = p0 + pr + i * PSTEP < pe;
-      raw[i] = 0;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const bool v = pv && gm + e < C;
-        raw[i] |= (unsigned)wq[v ? (long long)o * K + (long long)(gm + e) * KK + tap : 0]
-                  << (8 * e);
-        ok |= (v ? 1u : 0u) << (4 * i + e);
-      }
-    }
-  }
-  __device__ void stash(float* s, const float* tab) const {
-#pragma unroll
-    for (int i = 0; i < NQ; ++i) {
-      floatx4 v;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float x = tab[(raw[i] >> (8 * e)) & 255u];
-        v[e] = (ok >> (4 * i + e)) & 1u ? x : 0.0f;
-      }
-      *(floatx4*)&s[Lay::at(mq, pr + i * PSTEP)] = v;
-    }
-  }
-  __device__ void advance() {}
-};
-
-// B(p, col = (n, h, w)) = go'[n, o, h + PH - i*DH, w + PW - j*DW], KMajor
-// (quads of four pixels); go' = go * fp32(sx * sw[o]) when SCALED.
-template <int B, bool SCALED> struct DgradB {
-  using Lay = KMajor<B>;
-  static constexpr int QPR = B / 4, NQ = BK * B / (4 * GT), PSTEP = GT / QPR;
-  const float* go; atx_conv_geom g; int O, NHW;
-  const float* sx; const float* sw;
-  int jq, pr;
-  float sx0;
-  long long nb[4];          // go offset of image n_e (o = 0, h = w = 0); -1: no pixel
-  int hh[4], ww[4];         // pixel coordinates
-  floatx4 raw[NQ];
-  float sc[NQ];
-  unsigned ok;
-  __device__ void init(int t, int n0) {
-    jq = (t % QPR) * 4; pr = t / QPR;
-    if constexpr (SCALED) sx0 = sx[0];
-    const int HW = g.H * g.W;
-    const long long OHW = (long long)g.OH * g.OW;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int c = n0 + jq + e;
-      if (c < NHW) {
-        const int n = c / HW, hw = c - n * HW;
-        hh[e] = hw / g.W;
-        ww[e] = hw - hh[e] * g.W;
-        nb[e] = (long long)n * O * OHW;
-      } else {
-        nb[e] = -1; hh[e] = ww[e] = 0;
-      }
-    }
-  }
-  __device__ void fetch(int p0, int pe) {
-    const int tap = p0 / O;                   // uniform over the k-tile
-    const int o0 = p0 - tap * O;
-    const int ki = tap / g.KW, kj = tap - ki * g.KW;
-    const int dh0 = g.PH - ki * g.DH, dw0 = g.PW - kj * g.DW;
-    const long long OHW = (long long)g.OH * g.OW;
-    long long off[4];
-    bool pv[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int ih = hh[e] + dh0, iw = ww[e] + dw0;
-      pv[e] = nb[e] >= 0 && (unsigned)ih < (unsigned)g.OH && (unsigned)iw < (unsigned)g.OW;
-      off[e] = nb[e] + (long long)ih * g.OW + iw;
-    }
-    ok = 0;
-#pragma unroll
-    for (int i = 0; i < NQ; ++i) {
-      const int o = o0 + pr + i * PSTEP;
-      const bool rv = p0 + pr + i * PSTEP < pe;
-      if constexpr (SCALED) sc[i] = sw[rv ? o : 0];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const bool v = rv && pv[e];
-        raw[i][e] = go[v ? off[e] + (long long)o * OHW : 0];
-        ok |= (v ? 1u : 0u) << (4 * i + e);
-      }
-    }
-  }
-  __device__ void stash(float* s, const float*) const {
-#pragma unroll
-    for (int i = 0; i < NQ; ++i) {
-      floatx4 v;
-      float f = 1.0f;
-      if constexpr (SCALED) f = sx0 * sc[i];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float x = SCALED ? raw[i][e] * f : raw[i][e];
-        v[e] = (ok >> (4 * i + e)) & 1u ? x : 0.0f;
-      }
-      *(floatx4*)&s[Lay::at(jq, pr + i * PSTEP)] = v;
-    }
-  }
-  __device__ void advance() {}
-};
-
 // Rows r = n*L + l of the weight GEMM's contraction, tracked incrementally:
 // the thread's quad starts at r = p0 + pq and moves by BK per k-tile.
 struct RowCursor {
@@ -618,14 +501,12 @@ template <int B> struct WeightBRows {
 // 32): A(m = k, p = o).  Row m of a k-tile is 64 contiguous bytes per
 // plane; a thread copies 16-byte units (three planes, or only the h plane
 // when the table is bf16 exactly).  Buffer loads: rows past the planes read
-// 0.  DGRAD: rows m = input channel c of the implicit GEMM, whose k-tile
-// p0 holds tap t = p0 / O (O % 32 == 0): source row c*KK + t, columns from
-// p0 - t*O.
-template <int B, bool DGRAD> struct PlaneA {
+// 0.
+template <int B> struct PlaneA {
   static constexpr int NU = 3 * B * 4 / GT;   // 16-byte units per thread, three planes
   const uint16_t* planes; int pbytes;        // the planes and their size
   __amdgpu_buffer_rsrc_t res;
-  int Kp, Opad, KK, O, m0, t;
+  int Kp, Opad, m0, t;
   bool full;
   u32x4 raw[NU];
   __device__ void init(int tid, int mbase) {
@@ -633,15 +514,12 @@ template <int B, bool DGRAD> struct PlaneA {
     res = buffer_rsrc(planes, pbytes);
   }
   __device__ void fetch(int p0, int) {
-    int tap = 0, o0 = p0;
-    if constexpr (DGRAD) { tap = p0 / O; o0 = p0 - tap * O; }
 #pragma unroll
     for (int j = 0; j < NU; ++j) {
       if (j >= NU / 3 && !full) break;
       const int u = t + GT * j;
       const int q = u / (4 * B), row = (u >> 2) % B, unit = u & 3;
-      const int src = DGRAD ? (m0 + row) * KK + tap : m0 + row;
-      const unsigned off = (((unsigned)q * Kp + src) * Opad + o0 + 8 * unit) * 2u;
+      const unsigned off = (((unsigned)q * Kp + m0 + row) * Opad + p0 + 8 * unit) * 2u;
       raw[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(res, off, 0, 0));
     }
   }
@@ -711,77 +589,6 @@ template <int B, bool VEC, bool SCALED> struct GoCols {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         if (ob + i >= O) raw[i] = floatx4{0.f, 0.f, 0.f, 0.f};
-    }
-  }
-  template <bool FULL> __device__ void put(char* s, const uint2*) const {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      float v[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = SCALED ? raw[i][e] * sc[i] : raw[i][e];
-      uint2 P[3];
-      split4<FULL>(v, P);
-      put_parts<B, FULL>(s, 4 * cq + e, 4 * oq, P);
-    }
-  }
-  __device__ void advance() {}
-};
-
-// Implicit backward-data B: B(p = t*O + o, col = (n, h, w)) =
-// go'[n, o, h + PH - i*DH, w + PW - j*DW] (tap t = i*KW + j, uniform over a
-// k-tile since O % 32 == 0; zero outside go), with GoCols' thread layout
-// and scaling.  Elements outside the image use offset 2^31 (read 0).
-template <int B, bool SCALED> struct ShiftCols {
-  static_assert(B == 128, "ShiftCols covers 128 columns with 256 threads");
-  __amdgpu_buffer_rsrc_t res;
-  atx_conv_geom g; int O;
-  const float* sx; const float* sw;
-  int oq, cq;
-  int nb[4], hh[4], ww[4];  // image offset (elements, from the descriptor base; -1: none), pixel
-  floatx4 raw[4];
-  float sc[4];
-  __device__ void init(const float* go, long long go_elems, int tid, int n0, int NHW) {
-    oq = tid & 7; cq = tid >> 3;
-    const int HW = g.H * g.W;
-    const long long OHW = (long long)g.OH * g.OW;
-    const int nbase = n0 / HW;
-    const long long base = (long long)nbase * O * OHW;
-    const long long bytes = (go_elems - base) * 4;
-    res = buffer_rsrc(go + base, (int)(bytes < 0x7fffffffLL ? bytes : 0x7fffffffLL));
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int c = n0 + 4 * cq + e;
-      if (c < NHW) {
-        const int n = c / HW, hw = c - n * HW;
-        hh[e] = hw / g.W;
-        ww[e] = hw - hh[e] * g.W;
-        nb[e] = (int)((n - nbase) * O * OHW);
-      } else {
-        nb[e] = -1; hh[e] = ww[e] = 0;
-      }
-    }
-  }
-  __device__ void fetch(int p0, int) {
-    const int tap = p0 / O, o0 = p0 - tap * O;
-    const int ki = tap / g.KW, kj = tap - ki * g.KW;
-    const int dh0 = g.PH - ki * g.DH, dw0 = g.PW - kj * g.DW;
-    const int OHW = g.OH * g.OW;
-    unsigned off[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int ih = hh[e] + dh0, iw = ww[e] + dw0;
-      const bool v = nb[e] >= 0 && (unsigned)ih < (unsigned)g.OH && (unsigned)iw < (unsigned)g.OW;
-      off[e] = v ? (unsigned)(nb[e] + ih * g.OW + iw) * 4u : 0x80000000u;
-    }
-    const int ob = o0 + 4 * oq;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const unsigned ol = (unsigned)(ob + i) * OHW * 4u;
-      if constexpr (SCALED) sc[i] = sx[0] * sw[ob + i];
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        raw[i][e] = __builtin_bit_cast(
-            float, __builtin_amdgcn_raw_buffer_load_b32(res, off[e] + ol, 0, 0));
     }
   }
   template <bool FULL> __device__ void put(char* s, const uint2*) const {
@@ -1083,26 +890,6 @@ data_gemm_kernel(DataA<BM, VA> la, DataB<BN, VB, SC> lb, DataOut ep,
   data_epilogue<BM, BN, VB>(ep, acc, m0, n0);
 }
 
-// Implicit backward-data kernel: the data GEMM's epilogue (direct image
-// output with the optional fused STE) over DgradA x DgradB.
-template <int BM, int BN, bool SC, bool VO>
-__global__ void __launch_bounds__(GT, 2)
-dgrad_gemm_kernel(DgradA<BM> la, DgradB<BN, SC> lb, DataOut ep, const float* __restrict__ tx,
-                  int P) {
-  __shared__ float tab[256];
-  __shared__ __align__(16) float As[2][KMajor<BM>::SIZE];
-  __shared__ __align__(16) float Bs[2][KMajor<BN>::SIZE];
-  const int t = threadIdx.x;
-  tab[t] = tx[t];
-  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-  la.init(t, m0);
-  lb.init(t, n0);
-  __syncthreads();
-  floatx4 acc[BM / 32][BN / 32];
-  gemm_tiles<BM, BN, VO>(la, lb, tab, 0, P, acc, As[0], As[1], Bs[0], Bs[1]);
-  data_epilogue<BM, BN, VO>(ep, acc, m0, n0);
-}
-
 // planes[q][k][o] (q = h, m, l part of tx[wq[o*K + k]]; zero for k >= K or
 // o >= O) over Kp x Opad, the A operand of the plane data GEMMs.  A thread
 // writes eight consecutive o of one k per plane (16 bytes).
@@ -1139,7 +926,7 @@ weight_planes_kernel(const uint8_t* __restrict__ wq, const float* __restrict__ t
 // transposed epilogue.  Two blocks per CU.
 template <int BM, bool VB, bool SC>
 __global__ void __launch_bounds__(GT, 2)
-data_planes_kernel(PlaneA<BM, false> la, GoCols<128, VB, SC> lb, DataOut ep,
+data_planes_kernel(PlaneA<BM> la, GoCols<128, VB, SC> lb, DataOut ep,
                    const float* __restrict__ go, long long go_elems,
                    const float* __restrict__ tx, int O, int o_chunk) {
   __shared__ __align__(16) char As[Planes<BM>::SIZE];
@@ -1158,25 +945,312 @@ data_planes_kernel(PlaneA<BM, false> la, GoCols<128, VB, SC> lb, DataOut ep,
   data_epilogue<BM, 128, VB>(ep, acc, m0, n0);
 }
 
-// Implicit backward-data GEMM on split-bf16 planes (A rows c*KK + t of the
-// prepared planes, B = shifted go).  VO: 16-byte output stores.
-template <int BM, bool SC, bool VO>
-__global__ void __launch_bounds__(GT, 2)
-dgrad_planes_kernel(PlaneA<BM, true> la, ShiftCols<128, SC> lb, DataOut ep,
-                    const float* __restrict__ go, long long go_elems,
-                    const float* __restrict__ tx, int P) {
-  __shared__ __align__(16) char As[Planes<BM>::SIZE];
-  __shared__ __align__(16) char Bs[Planes<128>::SIZE];
+// -------------------------------- backward-data on position-major go planes
+// go' = go * fp32(sx * sw[o]) split once into bf16 parts, laid out for the
+// data GEMM's B operand: planes[p][ob][q][32] (p = n*L + l, ob = o / 32, part
+// q = h, m, l; zero for o >= O), 192 contiguous bytes per (p, ob).  Bound by
+// HBM: 4 bytes read and 6 written per element.  Block: 64 positions x 32
+// channels, transposed through LDS so that both sides are whole lines.
+__global__ void __launch_bounds__(256)
+go_planes_kernel(const float* __restrict__ go, int N, int O, int L, int nOb,
+                 const float* __restrict__ sx, const float* __restrict__ sw,
+                 uint16_t* __restrict__ planes) {
+  constexpr int ROW = 208;                 // LDS bytes per position (13 units: no conflicts)
+  __shared__ __align__(16) char tile[64 * ROW];
+  const int t = threadIdx.x, ob = blockIdx.y;
+  const int P = N * L;
+  const int pl = t & 63, o8 = (t >> 6) * 8;
+  const int p = blockIdx.x * 64 + pl;
+  if (p < P) {
+    const int n = p / L, l = p - n * L;
+    const float* src = go + (long long)n * O * L + l;
+    uint2 h[2][3];
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int o = ob * 32 + o8 + 4 * f + e;
+        v[e] = o < O ? src[(long long)o * L] : 0.0f;
+        if (sw && o < O) v[e] *= sx[0] * sw[o];
+      }
+      split4<true>(v, h[f]);
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      *(uint4*)(tile + pl * ROW + q * 64 + o8 * 2) =
+          make_uint4(h[0][q].x, h[0][q].y, h[1][q].x, h[1][q].y);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    const int u = t + 256 * j, row = u / 12, part = u - row * 12;
+    const long long pr = (long long)blockIdx.x * 64 + row;
+    if (pr < P)
+      *(uint4*)((char*)planes + (pr * nOb + ob) * 192 + part * 16) =
+          *(const uint4*)(tile + row * ROW + part * 16);
+  }
+}
+
+// Pixels of one residue class (h = ph mod SH, w = pw mod SW) of the image and
+// the taps that reach them: rows i0 + a*istep (a < nI), columns j0 + b*jstep
+// (b < nJ); pixel (ph + SH*hc, pw + SW*wc) reads output (hc + dh0 - a*dhs, wc
+// + dw0 - b*dws).  With stride 1 there is one class and every tap reaches it.
+struct TapClass {
+  int ph, pw, Hc, Wc;
+  int i0, istep, nI, j0, jstep, nJ;
+  int dh0, dhs, dw0, dws;
+};
+struct TapClasses { TapClass c[4]; int n; };
+
+// Image gradient gx[n][c][h][w] = sum over (tap, o) (before the STE): M = c,
+// columns = the pixels of a class (blockIdx.z / splits), contraction over the
+// class's taps and 32-channel blocks, split into `splits` partial images
+// (blockIdx.z % splits).  A = rows c*KK + tap of the weight planes, B = the go
+// planes' (shifted position, ob) rows, zero outside go.
+//
+// What bounded the kernel this replaces (go read, scaled and split in the
+// k-loop) was its loader: sixteen 4-byte loads with tap arithmetic, ~120 VALU
+// instructions and twelve LDS stores per thread and k-tile, against 48 MFMAs
+// per wave.  Both operands are now copied as they lie, by loads that write LDS
+// themselves (16 bytes a lane, no registers, no LDS store instructions) into
+// the second of two stages while the first is multiplied: one barrier per
+// k-tile.  A wave owns 32 rows x 64 columns; BM = 64: four waves, two blocks
+// per CU; BM = 128: eight waves share the columns' planes.
+struct TapArgs {
+  const uint16_t* wplanes; const uint16_t* gplanes;
+  int wbytes, gbytes;                      // sizes of the planes
+  int Kp, KK, nOb;                         // weight plane rows, taps, 32-channel blocks
+  int splits;
+  TapClasses classes;
+  atx_conv_geom g;
+};
+
+// One k-tile's planes of both operands.
+template <int BM> struct TapStage {
+  static constexpr int BYTES = Planes<BM>::SIZE + Planes<128>::SIZE;
+};
+
+using lds_ptr = __attribute__((address_space(3))) void*;
+
+// Copies for one k-tile: a wave's 1 KiB pieces are 16 rows of one plane.  Lane
+// i writes bytes 16 i of the piece, that is row s = 16 piece + i / 4 of the
+// plane in its stored order (Planes): source row r = s ^ ((s >> 2) & 1), unit
+// (i & 3) ^ ((s >> 1) & 3).
+template <int BM> struct TapLoader {
+  static constexpr int NW = BM / 16;       // waves
+  static constexpr int GB = 8 / NW;        // column pieces per wave
+  __amdgpu_buffer_rsrc_t wr, gr;
+  int a, b, ob;                            // tap (a, b) of the class, channel block
+  unsigned wrow, unit;                     // weight row (m0 + r) * KK, byte of the unit
+  int base[GB], hc[GB], wc[GB];            // image's first position, or -1; pixel
+  int wave;
+  bool full;
+  __device__ void init(const TapArgs& p, const TapClass& k, int m0, int n0, int cols, int tile,
+                       bool full_) {
+    wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    full = full_;
+    const int lane = threadIdx.x & 63, s = lane >> 2;          // within a piece
+    const int r = s ^ ((s >> 2) & 1);
+    unit = (unsigned)(((lane & 3) ^ ((s >> 1) & 3)) << 4);
+    wr = buffer_rsrc(p.wplanes, p.wbytes);
+    gr = buffer_rsrc(p.gplanes, p.gbytes);
+    const int tap = tile / p.nOb;
+    ob = tile - tap * p.nOb;
+    a = tap / k.nJ;
+    b = tap - a * k.nJ;
+    wrow = (unsigned)(m0 + 16 * wave + r) * p.KK;
+    const int HWc = k.Hc * k.Wc;
+#pragma unroll
+    for (int j = 0; j < GB; ++j) {
+      const int c = n0 + 16 * (wave + NW * j) + r;
+      const int n = c / HWc, q = c - n * HWc;
+      hc[j] = q / k.Wc;
+      wc[j] = q - hc[j] * k.Wc;
+      base[j] = c < cols ? n * p.g.OH * p.g.OW : -1;
+    }
+  }
+  // Issues the copies of the current k-tile into `st` and steps to the next.
+  __device__ __forceinline__ void load(const TapArgs& p, const TapClass& k, char* st) {
+    const int tap = (k.i0 + a * k.istep) * p.g.KW + k.j0 + b * k.jstep;
+    const unsigned woff = ((wrow + tap) * (unsigned)p.nOb + ob) * 64u + unit;
+    const int wplane = p.Kp * p.nOb * 64;
+    char* as = st + 1024 * wave;
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      if (q == 0 || full)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_ptr)(as + q * Planes<BM>::PLANE), 16,
+                                                 (int)woff, q * wplane, 0, 0);
+    const int dh = k.dh0 - a * k.dhs, dw = k.dw0 - b * k.dws;
+    char* bs = st + Planes<BM>::SIZE + 1024 * wave;
+#pragma unroll
+    for (int j = 0; j < GB; ++j) {
+      const int oh = hc[j] + dh, ow = wc[j] + dw;
+      const bool v = base[j] >= 0 && (unsigned)oh < (unsigned)p.g.OH &&
+                     (unsigned)ow < (unsigned)p.g.OW;
+      const unsigned off =
+          v ? (unsigned)((base[j] + oh * p.g.OW + ow) * p.nOb + ob) * 192u + unit : 0x80000000u;
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            gr, (lds_ptr)(bs + 1024 * NW * j + q * Planes<128>::PLANE), 16, (int)off, 64 * q, 0, 0);
+    }
+    if (++ob == p.nOb) {
+      ob = 0;
+      if (++b == k.nJ) { b = 0; ++a; }
+    }
+  }
+};
+
+// part += the k-tile's products for the wave's 32 rows x 64 columns (part
+// products smallest first, as mma_planes).
+template <int BM, bool EXACT, bool TR>
+__device__ __forceinline__ void mma_stage(const char* st, floatx4 (&part)[2][4]) {
+  constexpr int NA = EXACT ? 1 : 3;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int row = (wave >> 1) * 32 + (lane & 15), col = (wave & 1) * 64 + (lane & 15);
+  const int k8 = 8 * (lane >> 4);
+  const char* As = st;
+  const char* Bs = st + Planes<BM>::SIZE;
+  u32x4 a[NA][2];
+#pragma unroll
+  for (int q = 0; q < NA; ++q)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      a[q][i] = *(const u32x4*)(As + q * Planes<BM>::PLANE + Planes<BM>::at(row + 16 * i, k8));
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    u32x4 b[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      b[j] = *(const u32x4*)(Bs + q * Planes<128>::PLANE + Planes<128>::at(col + 16 * j, k8));
+#pragma unroll
+    for (int qa = EXACT ? 0 : 2 - q; qa >= 0; --qa)
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const bf16x8 x = __builtin_bit_cast(bf16x8, a[qa][i]);
+          const bf16x8 y = __builtin_bit_cast(bf16x8, b[j]);
+          part[i][j] = TR ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(y, x, part[i][j], 0, 0, 0)
+                          : __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, y, part[i][j], 0, 0, 0);
+        }
+  }
+}
+
+// acc += the products of `tiles` k-tiles.  A tap's sum, or at most FLUSH
+// k-tiles of it, is accumulated on its own and then added: one chain over all
+// taps and channels doubled the error of 9 x 128 terms against per-tap sums
+// (5.2e-7 against 2.0e-7 of the result).
+constexpr int FLUSH = 2;
+template <int BM, bool EXACT, bool TR>
+__device__ __forceinline__ void tap_sums(TapLoader<BM>& ld, const TapArgs& p, const TapClass& k,
+                                         int tiles, floatx4 (&acc)[2][4], char* st0, char* st1) {
+  floatx4 part[2][4];
+  int run = 0, ob = ld.ob;
+  ld.load(p, k, st0);
+  auto step = [&](char* cur, char* nxt, int left) __attribute__((always_inline)) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's copies are in LDS
+    __syncthreads();                                   // every wave's; the other stage is read
+    if (left > 1) ld.load(p, k, nxt);
+    if (run == 0) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) part[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    mma_stage<BM, EXACT, TR>(cur, part);
+    if (++ob == p.nOb) ob = 0;
+    if (++run == FLUSH || ob == 0 || left == 1) {
+      run = 0;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] += part[i][j];
+    }
+  };
+  for (; tiles > 1; tiles -= 2) {
+    step(st0, st1, tiles);
+    step(st1, st0, tiles - 1);
+  }
+  if (tiles > 0) step(st0, st1, tiles);
+}
+
+// VO: one class and H*W % 4 == 0 (transposed blocks, 16-byte stores).
+template <int BM, bool VO>
+__global__ void __launch_bounds__(BM * 4, BM == 64 ? 2 : 1)
+tap_planes_kernel(const TapArgs p, DataOut ep, const float* __restrict__ tx) {
+  __shared__ __align__(16) char st0[TapStage<BM>::BYTES];
+  __shared__ __align__(16) char st1[TapStage<BM>::BYTES];
   const int t = threadIdx.x;
+  const int ci = blockIdx.z / p.splits, sl = blockIdx.z - ci * p.splits;
+  const TapClass k = p.classes.c[ci];
+  const int cols = p.g.N * k.Hc * k.Wc;
   const int m0 = blockIdx.y * BM, n0 = blockIdx.x * 128;
-  la.init(t, m0);
-  lb.init(go, go_elems, t, n0, ep.NL);
-  const bool exact = table_exact(tx, t);
-  la.full = !exact;
-  floatx4 acc[BM / 32][4];
-  if (exact) gemm_planes<BM, 128, A_EXACT, VO>(la, lb, nullptr, 0, P, acc, As, Bs);
-  else gemm_planes<BM, 128, PROD6, VO>(la, lb, nullptr, 0, P, acc, As, Bs);
-  data_epilogue<BM, 128, VO>(ep, acc, m0, n0);
+  if (n0 >= cols) return;
+  const int tiles = k.nI * k.nJ * p.nOb;
+  const int chunk = (tiles + p.splits - 1) / p.splits;
+  const int tb = min(tiles, sl * chunk), te = min(tiles, tb + chunk);
+  ep.col += (long long)sl * ep.split_stride;
+  floatx4 acc[2][4];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  const bool exact = __syncthreads_or(t < 256 && bf16_rest(tx[t & 255]) != 0.0f) == 0;
+  if (tb < te) {
+    TapLoader<BM> ld;
+    ld.init(p, k, m0, n0, cols, tb, !exact);
+    if (exact) tap_sums<BM, true, VO>(ld, p, k, te - tb, acc, st0, st1);
+    else tap_sums<BM, false, VO>(ld, p, k, te - tb, acc, st0, st1);
+  }
+  // epilogue, with the fused STE (mask ? v : 0) / max(scale, 1e-12)
+  const int lane = t & 63, wave = t >> 6;
+  const int rb = m0 + (wave >> 1) * 32, cb = n0 + (wave & 1) * 64;
+  const float sdiv = ep.mask ? fmaxf(ep.scale[0], 1e-12f) : 1.0f;
+  if constexpr (VO) {                      // lane: columns c .. c + 3 of one row per block
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int c = cb + 16 * j + 4 * (lane >> 4);
+      if (c >= cols) continue;
+      const int n = c / ep.L;
+      const long long off = (long long)n * ep.K * ep.L + (c - n * ep.L);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int m = rb + 16 * i + (lane & 15);
+        if (m >= ep.K) continue;
+        const long long at = off + (long long)m * ep.L;
+        floatx4 v = acc[i][j];
+        if (ep.mask) {
+          const unsigned mk = *(const unsigned*)(ep.mask + at);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = ((mk >> (8 * e)) & 255u ? v[e] : 0.0f) / sdiv;
+        }
+        *(floatx4*)(ep.col + at) = v;
+      }
+    }
+  } else {                                 // lane: rows m .. m + 3 of one column per block
+    const int HWc = k.Hc * k.Wc;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int c = cb + 16 * j + (lane & 15);
+      if (c >= cols) continue;
+      const int n = c / HWc, q = c - n * HWc;
+      const int hc = q / k.Wc, wc = q - hc * k.Wc;
+      const long long off = (long long)n * ep.K * ep.L +
+                            (long long)(k.ph + p.g.SH * hc) * p.g.W + k.pw + p.g.SW * wc;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int m = rb + 16 * i + 4 * (lane >> 4) + e;
+          if (m >= ep.K) continue;
+          const long long at = off + (long long)m * ep.L;
+          const float v = acc[i][j][e];
+          ep.col[at] = ep.mask ? (ep.mask[at] ? v : 0.0f) / sdiv : v;
+        }
+    }
+  }
 }
 
 template <class LB> __device__ __forceinline__ void set_pad(LB&, const float*) {}
@@ -1381,7 +1455,7 @@ static void launch_data(const DataArgs& a, hipStream_t stream) {
 template <int BM, bool VB, bool SC>
 static void launch_data_planes(const DataArgs& a, hipStream_t stream) {
   const int NL = a.N * a.L;
-  PlaneA<BM, false> la{};
+  PlaneA<BM> la{};
   la.planes = a.planes; la.pbytes = (int)weight_planes_bytes(a.K, a.O);
   la.Kp = (int)(cdiv(a.K, 128) * 128); la.Opad = (int)(cdiv(a.O, BK) * BK);
   GoCols<128, VB, SC> lb{};
@@ -1512,62 +1586,166 @@ static void dispatch_weight_rows(const float* go, const uint16_t* xt, long long 
 #undef ATX_LWR
 }
 
-template <int BM, bool SC>
-static int launch_dgrad(const float* go, const uint8_t* wq, const float* tx,
-                        const atx_conv_geom& g, int O, const float* sx, const float* sw,
-                        const uint8_t* mask, const float* scale, float* gx, uint16_t* planes,
-                        hipStream_t stream) {
-  constexpr int BN = 128;
-  const int KK = g.KH * g.KW, K = g.C * KK, HW = g.H * g.W, NHW = g.N * HW;
-  const bool vo = HW % 4 == 0 && (uintptr_t)gx % 16 == 0 && (uintptr_t)mask % 4 == 0;
-  if (planes && planes_fit(HW, O, (long long)g.OH * g.OW)) {
-    int rc = launch_weight_planes(wq, tx, O, K, planes, stream);
-    if (rc) return rc;
-    PlaneA<BM, true> la{};
-    la.planes = planes; la.pbytes = (int)weight_planes_bytes(K, O);
-    la.Kp = (int)(cdiv(K, 128) * 128); la.Opad = O; la.KK = KK; la.O = O;
-    ShiftCols<BN, SC> lb{};
-    lb.g = g; lb.O = O; lb.sx = sx; lb.sw = sw;
-    DataOut ep{gx, g.C, HW, NHW, mask, scale, 0};
-    dim3 grid((unsigned)cdiv(NHW, BN), (unsigned)cdiv(g.C, BM), 1);
-    const long long go_elems = (long long)g.N * O * g.OH * g.OW;
-    if (vo)
-      hipLaunchKernelGGL((dgrad_planes_kernel<BM, SC, true>), grid, dim3(GT), 0, stream, la, lb,
-                         ep, go, go_elems, tx, KK * O);
-    else
-      hipLaunchKernelGGL((dgrad_planes_kernel<BM, SC, false>), grid, dim3(GT), 0, stream, la,
-                         lb, ep, go, go_elems, tx, KK * O);
-    return check_launch("dgrad_planes_kernel");
-  }
-  DgradA<BM> la{};
-  la.wq = wq; la.K = K; la.KK = KK; la.C = g.C; la.O = O;
-  DgradB<BN, SC> lb{};
-  lb.go = go; lb.g = g; lb.O = O; lb.NHW = NHW; lb.sx = sx; lb.sw = sw;
-  DataOut ep{gx, g.C, HW, NHW, mask, scale, 0};
-  dim3 grid((unsigned)cdiv(NHW, BN), (unsigned)cdiv(g.C, BM), 1);
-  if (vo)
-    hipLaunchKernelGGL((dgrad_gemm_kernel<BM, BN, SC, true>), grid, dim3(GT), 0, stream, la, lb,
-                       ep, tx, KK * O);
-  else
-    hipLaunchKernelGGL((dgrad_gemm_kernel<BM, BN, SC, false>), grid, dim3(GT), 0, stream, la,
-                       lb, ep, tx, KK * O);
-  return check_launch("dgrad_gemm_kernel");
+// Residue classes of a stride of 1 or 2 per axis, most taps first.
+static TapClasses tap_classes(const atx_conv_geom& g) {
+  TapClasses t{};
+  const auto axis = [](int r, int S, int K, int Pd, int D, int size, int& i0, int& istep, int& nI,
+                       int& d0, int& ds, int& ext) {
+    ext = size > r ? (size - r + S - 1) / S : 0;
+    nI = 0;
+    istep = S == 2 && (D & 1) ? 2 : 1;     // taps of one parity of i*D
+    i0 = 0;
+    for (int i = 0; i < K; ++i)
+      if ((r + Pd - i * D) % S == 0) { if (nI++ == 0) i0 = i; }
+    d0 = (r + Pd - i0 * D) / S;            // exact for a reaching tap
+    ds = istep * D / S;
+  };
+  for (int ph = 0; ph < g.SH; ++ph)
+    for (int pw = 0; pw < g.SW; ++pw) {
+      TapClass c{};
+      c.ph = ph; c.pw = pw;
+      axis(ph, g.SH, g.KH, g.PH, g.DH, g.H, c.i0, c.istep, c.nI, c.dh0, c.dhs, c.Hc);
+      axis(pw, g.SW, g.KW, g.PW, g.DW, g.W, c.j0, c.jstep, c.nJ, c.dw0, c.dws, c.Wc);
+      int at = t.n++;
+      for (; at > 0 && t.c[at - 1].nI * t.c[at - 1].nJ < c.nI * c.nJ; --at) t.c[at] = t.c[at - 1];
+      t.c[at] = c;
+    }
+  return t;
 }
 
-// The implicit backward-data GEMM serves stride-1 convs whose O fills whole
-// k-tiles (one tap per tile) and whose C x N*H*W output tiles fill the GPU
-// (>= 512 blocks); 1x1 unpadded convs take the direct path.  With fewer
-// tiles the col GEMM (M = C*KH*KW) plus col2im is faster: measured on the
-// ResNet-50 3x3 layers at batch 64, a split implicit GEMM took 241 us where
-// the col path takes 198 us (14x14) and 214 us (7x7); at 28x28 (392 tiles)
-// the implicit GEMM takes 255 us against 221 us; at 56x56 the unsplit
-// implicit GEMM takes 262-290 us against 462 us.
-static bool implicit_dgrad(const atx_conv_geom& g, int O) {
-  const long long tiles = cdiv((long long)g.N * g.H * g.W, 128) * cdiv(g.C, tile_of(g.C));
-  return g.SH == 1 && g.SW == 1 && O % BK == 0 && O > 0 && tiles >= 512 &&
-         !(g.KH == 1 && g.KW == 1 && g.PH == 0 && g.PW == 0) &&
-         (long long)g.N * g.C * g.H * g.W < 0x7fffffffLL &&
-         (long long)g.KH * g.KW * O < 0x7fffffffLL;
+static long long go_planes_bytes(long long P, int O) { return P * cdiv(O, BK) * 192; }
+
+// Split of the tap GEMM's contraction (partial images summed by split_sum):
+// the cost of data_splits over the tiles and the deepest class's k-tiles.
+static int tap_splits(const atx_conv_geom& g, int O) {
+  const TapClasses t = tap_classes(g);
+  const long long numel = (long long)g.N * g.C * g.H * g.W;
+  const long long mt = cdiv(g.C, 64), nob = cdiv(O, BK);
+  const long long kt = (long long)t.c[0].nI * t.c[0].nJ * nob;
+  double work = 0.0;                       // k-tiles of all blocks
+  long long blocks = 0;
+  for (int i = 0; i < t.n; ++i) {
+    const long long b = cdiv((long long)g.N * t.c[i].Hc * t.c[i].Wc, 128) * mt;
+    blocks += b;
+    work += (double)b * t.c[i].nI * t.c[i].nJ * nob;
+  }
+  const long long smax = std::max<long long>(1, std::min<long long>(kt / 4, 64));
+  double best = 0.0;
+  long long pick = 1;
+  for (long long s = 1; s <= smax; ++s) {
+    const double rounds = std::max((double)cdiv(blocks * s, 512) * 4.0 + work / 512.0,
+                                   (double)cdiv(kt, s) + 4.0);
+    const double idle = (double)cdiv(blocks * s, 512) * 512.0 / (blocks * s);
+    const double cost = rounds * (t.n == 1 ? idle : 1.0) +
+                        (s > 1 ? 2.0 + (double)s * numel / 1.5e6 : 0.0);
+    if (s == 1 || cost < best) { best = cost; pick = s; }
+  }
+  return (int)pick;
+}
+
+// Images per pass of the tap GEMM (32-bit plane offsets, pixel counts and
+// output indices), 0 when one image does not fit.
+static int tap_images(const atx_conv_geom& g, int O) {
+  const long long L = (long long)g.OH * g.OW, HW = (long long)g.H * g.W;
+  const long long lim = 0x7fffffffLL - 4096;
+  const long long n = std::min(std::min(lim / go_planes_bytes(L, O), lim / (HW * g.C)), lim / HW);
+  return (int)std::min<long long>(n, g.N);
+}
+
+// 1e8 products, or (stride 1) 512 output tiles: a large image of few channels.
+static bool tap_size(const atx_conv_geom& g, int O) {
+  const double K = (double)g.C * g.KH * g.KW, P = (double)g.N * g.OH * g.OW;
+  return P * O * K >= 1e8 ||
+         (g.SH == 1 && g.SW == 1 && (double)g.N * g.H * g.W * cdiv(g.C, 64) >= 512 * 128);
+}
+
+// The tap GEMM serves convs of at least two taps, strides of 1 or 2 and
+// tap_size().  A 1x1 conv's columns are its gradient, or (stride 2) most of its
+// pixels have no tap: the column GEMM there reads go once per 128 rows and
+// writes the result, which the go planes' pass does not beat (1024 -> 256 at
+// 14 x 14, batch 64: 74 against 85 us).  Below 1e8 products the extra launch
+// costs more than the loop saves (1.8e6 to 5.5e6 products: 14-18 us against
+// 17-19; 3e8: 27.5 against 24.6).  Above, on the 3x3 layers of ResNet-50 at
+// batch 64 and ResNet-18 at 128 with LRE tables, against the column GEMM plus
+// col2im or the implicit GEMM that read go itself: 56 x 56 x 64 186 -> 140 us,
+// 28 x 28 x 128 191 -> 130, 14 x 14 x 256 144 -> 133, 7 x 7 x 512 143 -> 122,
+// stride 2 at 56 x 56 x 128 256 -> 206, 16 x 16 x 128 126 -> 79; with a
+// bf16-exact (STE) table 159 -> 89 and 106 -> 54 at 28 x 28 and 16 x 16.
+static bool tap_gemm(const atx_conv_geom& g, int O) {
+  const long long K = (long long)g.C * g.KH * g.KW, L = (long long)g.OH * g.OW;
+  return g.KH * g.KW > 1 && (g.SH == 1 || g.SH == 2) && (g.SW == 1 || g.SW == 2) && O > 0 &&
+         g.N > 0 && K > 0 && L > 0 && g.H > 0 && g.W > 0 &&
+         tap_size(g, O) && weight_planes_bytes((int)K, O) < 0x7fffffffLL &&
+         (double)g.KH * g.KW * cdiv(O, BK) < 1e8 && cdiv(g.C, 64) <= 65535 &&
+         cdiv(O, BK) <= 65535 && tap_images(g, O) > 0;
+}
+
+// Workspace of one pass: [weight planes][go planes][split partials].
+static long long tap_workspace_bytes(const atx_conv_geom& g, int O) {
+  const int S = tap_splits(g, O);
+  return weight_planes_bytes(g.C * g.KH * g.KW, O) +
+         (go_planes_bytes((long long)g.N * g.OH * g.OW, O) + 255) / 256 * 256 +
+         (S > 1 ? (long long)S * g.N * g.C * g.H * g.W * 4 : 0);
+}
+
+static int run_tap_images(const float* go, const uint8_t* wq, const float* tx,
+                        const atx_conv_geom& g, int O, const float* sx, const float* sw,
+                        const uint8_t* mask, const float* scale, float* gx, char* ws,
+                        hipStream_t stream) {
+  const int KK = g.KH * g.KW, K = g.C * KK, L = g.OH * g.OW, P = g.N * L, HW = g.H * g.W;
+  const int nob = (int)cdiv(O, BK), S = tap_splits(g, O);
+  uint16_t* wplanes = (uint16_t*)ws;
+  uint16_t* gplanes = (uint16_t*)(ws + weight_planes_bytes(K, O));
+  float* partials = (float*)((char*)gplanes + (go_planes_bytes(P, O) + 255) / 256 * 256);
+  int rc = launch_weight_planes(wq, tx, O, K, wplanes, stream);
+  if (rc) return rc;
+  hipLaunchKernelGGL(go_planes_kernel, dim3((unsigned)cdiv(P, 64), (unsigned)nob), dim3(256), 0,
+                     stream, go, g.N, O, L, nob, sx, sw, gplanes);
+  rc = check_launch("go_planes_kernel");
+  if (rc) return rc;
+  const TapClasses classes = tap_classes(g);
+  const bool split = S > 1;
+  float* out = split ? partials : gx;
+  const long long numel = (long long)g.N * g.C * HW;
+  DataOut ep{out, g.C, HW, g.N * HW, split ? nullptr : mask, split ? nullptr : scale, numel};
+  TapArgs p{};
+  p.wplanes = wplanes; p.gplanes = gplanes;
+  p.wbytes = (int)weight_planes_bytes(K, O); p.gbytes = (int)go_planes_bytes(P, O);
+  p.Kp = (int)(cdiv(K, 128) * 128); p.KK = KK; p.nOb = nob;
+  p.splits = S; p.classes = classes; p.g = g;
+  const bool vo = classes.n == 1 && HW % 4 == 0 && (uintptr_t)out % 16 == 0 &&
+                  (split || (uintptr_t)mask % 4 == 0);
+  long long ct = 0;
+  for (int i = 0; i < classes.n; ++i)
+    ct = std::max(ct, cdiv((long long)g.N * classes.c[i].Hc * classes.c[i].Wc, 128));
+  const auto launch = [&](auto bm) {
+    constexpr int BM = decltype(bm)::value;
+    const dim3 grid((unsigned)ct, (unsigned)cdiv(g.C, BM), (unsigned)(classes.n * S));
+    if (vo)
+      hipLaunchKernelGGL((tap_planes_kernel<BM, true>), grid, dim3(BM * 4), 0, stream, p, ep, tx);
+    else
+      hipLaunchKernelGGL((tap_planes_kernel<BM, false>), grid, dim3(BM * 4), 0, stream, p, ep, tx);
+  };
+  if (g.C <= 64) launch(std::integral_constant<int, 64>{});
+  else launch(std::integral_constant<int, 128>{});
+  rc = check_launch("tap_planes_kernel");
+  if (rc || !split) return rc;
+  return launch_split_sum(partials, S, numel, (int)numel, mask, scale, gx, stream);
+}
+
+// All images, in passes of at most tap_images().
+static int run_tap_gemm(const float* go, const uint8_t* wq, const float* tx, atx_conv_geom g,
+                        int O, const float* sx, const float* sw, const uint8_t* mask,
+                        const float* scale, float* gx, char* ws, hipStream_t stream) {
+  const int N = g.N, step = tap_images(g, O);
+  const long long gi = (long long)O * g.OH * g.OW, xi = (long long)g.C * g.H * g.W;
+  for (int n = 0; n < N; n += step) {
+    g.N = std::min(step, N - n);
+    const int rc = run_tap_images(go + n * gi, wq, tx, g, O, sx, sw, mask ? mask + n * xi : nullptr,
+                                  scale, gx + n * xi, ws, stream);
+    if (rc) return rc;
+  }
+  return ATX_OK;
 }
 
 }  // namespace atx
@@ -1600,12 +1778,21 @@ static bool direct_columns(const atx_conv_geom& g) {
 }
 
 // Workspace of atx_conv_bwd_data: [bf16 weight planes][split partials][col
-// (unless direct or implicit)].
+// (unless direct)], or the tap GEMM's (tap_workspace_bytes).
 long long atx_conv_bwd_data_workspace_bytes(atx_conv_geom g, int O) {
   const int K = g.C * g.KH * g.KW, L = g.OH * g.OW;
   if (g.N <= 0 || K <= 0 || L <= 0 || O <= 0) return 0;
   const long long planes = weight_planes_bytes(K, O);
-  if (implicit_dgrad(g, O)) return planes;
+  if (tap_gemm(g, O)) {
+    atx_conv_geom part = g;                // a pass, and the last, smaller one
+    part.N = tap_images(g, O);
+    long long bytes = tap_workspace_bytes(part, O);
+    if (g.N % part.N) {
+      part.N = g.N % part.N;
+      bytes = std::max(bytes, tap_workspace_bytes(part, O));
+    }
+    return bytes;
+  }
   const long long numel = (long long)g.N * K * L;
   const int S = data_splits(g.N, O, K, L);
   return planes + ((S > 1 ? S : 0) + (direct_columns(g) ? 0 : 1)) * numel * 4;
@@ -1632,15 +1819,9 @@ int atx_conv_bwd_data(const float* go, const uint8_t* wq, const float* tx, atx_c
     planes = (uint16_t*)workspace;
     rest = (float*)((char*)workspace + weight_planes_bytes(K, O));
   }
-  if (L > 0 && implicit_dgrad(g, O)) {
+  if (tap_gemm(g, O)) {
     ATX_REQUIRE(go && wq && tx, "atx_conv_bwd_data: null pointer");
-    ATX_REQUIRE(cdiv(g.C, 64) <= 65535, "atx_conv_bwd_data: too many channels");
-    const bool sc = go_sw != nullptr;
-#define ATX_LD(M_, S_) \
-  launch_dgrad<M_, S_>(go, wq, tx, g, O, go_sx, go_sw, mask, scale, gx, planes, stream)
-    if (tile_of(g.C) == 64) return sc ? ATX_LD(64, true) : ATX_LD(64, false);
-    return sc ? ATX_LD(128, true) : ATX_LD(128, false);
-#undef ATX_LD
+    return run_tap_gemm(go, wq, tx, g, O, go_sx, go_sw, mask, scale, gx, (char*)workspace, stream);
   }
   const long long numel = (long long)g.N * K * L;
   const int S = (O > 0 && numel > 0) ? data_splits(g.N, O, K, L) : 1;

@@ -506,11 +506,12 @@ int atx_conv_bwd_data_col(const float* go, const uint8_t* wq, const float* tx,
 /* Image gradient of the conv: col as above (with the go scale), folded into
  * gx [N,C,H,W] with the per-tensor fake-quant STE fused when mask != NULL:
  * gx = (mask ? g : 0) / max(scale[0], 1e-12).  A 1x1 stride-1 unpadded conv
- * writes gx straight from the GEMM, and so does a stride-1 conv with
- * O % 32 == 0 whose C x N*H*W output fills >= 512 tiles (implicit GEMM over
- * (tap, o)); otherwise the workspace holds col.  When the output tiles
- * cannot fill the GPU the contraction over O is split into partial slices
- * (in the workspace) summed in a fixed order.  The workspace also holds the
+ * writes gx straight from the GEMM, and so does a conv of two taps or more,
+ * strides of 1 or 2 and enough work (an implicit GEMM over (tap, o) on go
+ * split into bf16 planes, which the workspace holds; a batch whose planes
+ * exceed 2 GiB takes several passes); otherwise the workspace holds col.
+ * When the output tiles cannot fill the GPU the contraction is split into
+ * partial slices (in the workspace) summed in a fixed order.  The workspace also holds the
  * tx[wq] values as bf16 parts for the matrix cores (the products are the
  * fp32 products to within 2^-20 relative; exact when tx holds bf16 values,
  * as the STE's integers do).  Size: atx_conv_bwd_data_workspace_bytes(g, O),
