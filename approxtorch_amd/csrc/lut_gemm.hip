@@ -142,79 +142,21 @@ __global__ void lut_prepare_kernel(const float* __restrict__ lut,
 
 // ------------------------------------------------------------- operand pack
 // xt[slot][r] = row_offset(x[n][operand_tap(slot, r)][l]) for r < R
-// (r = n*L + l); 0 for r >= R and taps >= K.  A thread writes the four rows
-// of a quad (one tap) as one 8-byte store; when L % 4 == 0 the quad is four
-// consecutive elements of one x row, read with one 4- (u8) or 16-byte (fp32)
-// load (`vec`: L % 4 == 0 and the pointers aligned for it).  The grid stride over quads is a multiple of 4, so every thread keeps
-// one tap per slot.
+// (r = n*L + l); 0 for r >= R and taps >= K.  The four rows of a quad (one tap)
+// are one 8-byte store; when L % 4 == 0 the quad is four consecutive elements
+// of one x row, read with one 4- (u8) or 16-byte (fp32) load (`vec`: L % 4 ==
+// 0 and the pointers aligned for it).
+//
+// A thread owns one quad of rows and one quad of slots (blockIdx.y = slot
+// quad): the four taps' loads are in flight together and go out as four
+// 8-byte pieces.  Bound by HBM: 4 (fp32) or 1 byte read, 2 written per element
+// and 1 more for the fp32 operand's index image.  16 x 1152 x 784 fp32: 52 us
+// with one tap per thread, 27 us now (3.7 TB/s); the u8 operand 3.6 -> 6 TB/s.
 template <typename T>
-__global__ void pack_x_kernel(const T* __restrict__ x, int N, int K, int L,
-                              int offset, uint8_t* __restrict__ xq,
-                              uint16_t* __restrict__ xt, int Rpad, bool vec,
-                              int* __restrict__ upper) {
-  const int R = N * L;
-  const int q0 = blockIdx.x * blockDim.x + threadIdx.x;
-  const int qstride = gridDim.x * blockDim.x;
-  const int nquad = Rpad >> 2;
-  bool low = false;             // some index of rows < R and taps < K is < 128
-  for (int slot = blockIdx.y; slot < operand_rows(K); slot += gridDim.y) {
-    const int k = operand_tap(slot, q0 << 2);
-    uint16_t* dst = xt + (long long)slot * Rpad;
-    for (int q = q0; q < nquad; q += qstride) {
-      const int r0 = q << 2;
-      unsigned v[4] = {0u, 0u, 0u, 0u};
-      bool any = false;
-      if (k < K && r0 < R) {
-        any = true;
-        int n = r0 / L;
-        int l = r0 - n * L;
-        if (vec) {
-          const long long src = ((long long)n * K + k) * L + l;
-          if constexpr (sizeof(T) == 4) {
-            const float4 f = *(const float4*)(x + src);
-            v[0] = quant_index(f.x, offset); v[1] = quant_index(f.y, offset);
-            v[2] = quant_index(f.z, offset); v[3] = quant_index(f.w, offset);
-            if (xq) *(uchar4*)(xq + src) = make_uchar4(v[0], v[1], v[2], v[3]);
-          } else {
-            const unsigned w = *(const unsigned*)(x + src);
-            v[0] = w & 255u; v[1] = (w >> 8) & 255u; v[2] = (w >> 16) & 255u; v[3] = w >> 24;
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            if (r0 + e < R) {
-              const long long src = ((long long)n * K + k) * L + l;
-              if constexpr (sizeof(T) == 4) {
-                v[e] = quant_index((float)x[src], offset);
-                if (xq) xq[src] = (uint8_t)v[e];
-              } else {
-                v[e] = (unsigned)x[src];
-              }
-            }
-            if (++l == L) { l = 0; ++n; }
-          }
-        }
-      }
-      unsigned off[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const bool live = any && r0 + e < R;
-        off[e] = live ? row_offset(v[e]) : 0u;
-        low |= live && v[e] < 128u;
-      }
-      *(uint2*)(dst + r0) = make_uint2(off[0] | (off[1] << 16), off[2] | (off[3] << 16));
-    }
-  }
-  if (upper && low) upper[0] = 0;        // benign race: every writer stores 0
-}
-
-// u8 row operand with one quad of rows and one quad of slots per thread
-// (blockIdx.y = slot quad): the four taps' bytes of the quad are read
-// together (one 4-byte load each when `vec`, as in pack_x_kernel) and
-// written as four 8-byte pieces, so every thread moves 16 elements.
 __global__ void __launch_bounds__(256)
-pack_x_u8_quads_kernel(const uint8_t* __restrict__ x, int N, int K, int L,
-                       uint16_t* __restrict__ xt, int Rpad, bool vec, int* __restrict__ upper) {
+pack_x_quads_kernel(const T* __restrict__ x, int N, int K, int L, int offset,
+                    uint8_t* __restrict__ xq, uint16_t* __restrict__ xt, int Rpad, bool vec,
+                    int* __restrict__ upper) {
   const int q = blockIdx.x * 256 + threadIdx.x;
   if (q >= (Rpad >> 2)) return;
   const int R = N * L;
@@ -234,36 +176,71 @@ pack_x_u8_quads_kernel(const uint8_t* __restrict__ x, int N, int K, int L,
 #pragma unroll
     for (int e = 0; e < 4; ++e) base[e] = 0;
   }
-  const int k4 = blockIdx.y * 4;
-  unsigned v[4];
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int k = k4 | ((q + u) & 3);            // this quad's tap of slot k4 + u
-    const long long kl = (long long)min(k, K - 1) * L;
-    if (vec) {
-      v[u] = (k < K && valid) ? *(const unsigned*)(x + base[0] + kl) : 0u;
-    } else {
-      v[u] = 0;
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (k < K && ((valid >> e) & 1u)) v[u] |= (unsigned)x[base[e] + kl] << (8 * e);
-    }
-  }
-  uint16_t* dst = xt + (long long)k4 * Rpad + r0;
   bool low = false;             // some index of rows < R and taps < K is < 128
+  for (int k4 = blockIdx.y * 4; k4 < K; k4 += gridDim.y * 4) {
+    unsigned v[4];                                 // the taps' four indices, a byte each
+    if constexpr (sizeof(T) == 4) {
+      float f[4][4];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    const int k = k4 | ((q + u) & 3);
-    unsigned off[4];
+      for (int u = 0; u < 4; ++u) {
+        const int k = k4 | ((q + u) & 3);          // this quad's tap of slot k4 + u
+        const long long kl = (long long)min(k, K - 1) * L;
+        if (vec) {
+          float4 w = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+          if (k < K && valid) w = *(const float4*)(x + base[0] + kl);
+          f[u][0] = w.x; f[u][1] = w.y; f[u][2] = w.z; f[u][3] = w.w;
+        } else {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const bool live = k < K && ((valid >> e) & 1u);
-      const unsigned idx = (v[u] >> (8 * e)) & 255u;
-      off[e] = live ? row_offset(idx) : 0u;
-      low |= live && idx < 128u;
+          for (int e = 0; e < 4; ++e) f[u][e] = k < K && ((valid >> e) & 1u) ? x[base[e] + kl] : 0.0f;
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        v[u] = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[u] |= quant_index(f[u][e], offset) << (8 * e);
+        const int k = k4 | ((q + u) & 3);
+        if (xq && k < K && valid) {
+          const long long kl = (long long)k * L;
+          if (vec) {
+            *(unsigned*)(xq + base[0] + kl) = v[u];
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if ((valid >> e) & 1u) xq[base[e] + kl] = (uint8_t)(v[u] >> (8 * e));
+          }
+        }
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int k = k4 | ((q + u) & 3);
+        const long long kl = (long long)min(k, K - 1) * L;
+        if (vec) {
+          v[u] = (k < K && valid) ? *(const unsigned*)(x + base[0] + kl) : 0u;
+        } else {
+          v[u] = 0;
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (k < K && ((valid >> e) & 1u)) v[u] |= (unsigned)x[base[e] + kl] << (8 * e);
+        }
+      }
     }
-    *(uint2*)(dst + (long long)u * Rpad) =
-        make_uint2(off[0] | (off[1] << 16), off[2] | (off[3] << 16));
+    uint16_t* dst = xt + (long long)k4 * Rpad + r0;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int k = k4 | ((q + u) & 3);
+      unsigned off[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const bool live = k < K && ((valid >> e) & 1u);
+        const unsigned idx = (v[u] >> (8 * e)) & 255u;
+        off[e] = live ? row_offset(idx) : 0u;
+        low |= live && idx < 128u;
+      }
+      *(uint2*)(dst + (long long)u * Rpad) =
+          make_uint2(off[0] | (off[1] << 16), off[2] | (off[3] << 16));
+    }
   }
   if (upper && low) upper[0] = 0;        // benign race: every writer stores 0
 }
@@ -1075,12 +1052,12 @@ int atx_pack_x_f32(const float* x, int N, int K, int L, int offset, uint8_t* xq,
   if ((long long)K * Rpad == 0) return ATX_OK;
   // an empty x (N*L == 0) only writes the zero padding rows
   ATX_REQUIRE(xt && ((long long)N * L == 0 || x), "atx_pack_x_f32: null pointer");
-  dim3 grid((unsigned)std::min<long long>(cdiv(Rpad / 4, 256), 1024),
-            (unsigned)std::min(operand_rows(K), 65535));
+  const dim3 grid((unsigned)cdiv(Rpad / 4, 256),
+                  (unsigned)std::min(operand_rows(K) / 4, 65535));
   const bool vec = L % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)xq % 4 == 0;
-  hipLaunchKernelGGL(pack_x_kernel<float>, grid, dim3(256), 0, stream, x, N, K, L,
+  hipLaunchKernelGGL(pack_x_quads_kernel<float>, grid, dim3(256), 0, stream, x, N, K, L,
                      offset, xq, xt, Rpad, vec, upper);
-  return check_launch("pack_x_kernel<float>");
+  return check_launch("pack_x_quads_kernel<float>");
 }
 
 int atx_pack_x_u8(const uint8_t* xq, int N, int K, int L, uint16_t* xt, int Rpad,
@@ -1093,9 +1070,9 @@ int atx_pack_x_u8(const uint8_t* xq, int N, int K, int L, uint16_t* xt, int Rpad
   ATX_REQUIRE(operand_rows(K) / 4 <= 65535, "atx_pack_x_u8: K too large");
   const dim3 grid((unsigned)cdiv(Rpad / 4, 256), (unsigned)(operand_rows(K) / 4));
   const bool vec = L % 4 == 0 && (uintptr_t)xq % 4 == 0;
-  hipLaunchKernelGGL(pack_x_u8_quads_kernel, grid, dim3(256), 0, stream, xq, N, K, L, xt, Rpad,
-                     vec, upper);
-  return check_launch("pack_x_u8_quads_kernel");
+  hipLaunchKernelGGL(pack_x_quads_kernel<uint8_t>, grid, dim3(256), 0, stream, xq, N, K, L, 0,
+                     (uint8_t*)nullptr, xt, Rpad, vec, upper);
+  return check_launch("pack_x_quads_kernel<u8>");
 }
 
 int atx_pack_w_f32(const float* w, int O, int K, int offset, uint8_t* wq,

@@ -40,9 +40,7 @@ def _gemm_grads(go, xq, wq, tx, tw):
     O = wq.size(0)
     g = _gemm_geom(N, K, L)
     go = go.contiguous()
-    col = torch.empty((N, K, L), dtype=torch.float32, device=go.device)
-    ops.L.call("atx_conv_bwd_data_col", go.data_ptr(), wq.data_ptr(), tx.data_ptr(), N, O, K,
-               L, col.data_ptr(), ops.L.stream_of(go))
+    col = ops.gemm_backward_data(go, wq, tx)
     gw = ops.conv_backward_weight(go, xq.view(N, K, 1, L), tw, g, O, 128)
     return col, gw
 
