@@ -149,3 +149,20 @@ def test_gemm2d_degenerate_and_invalid():
                                   torch.zeros(5, 7, device=DEV), lut)
     with pytest.raises(RuntimeError):
         ops.gemm_fake_int8_claude(torch.zeros(4, 5), torch.zeros(5, 7), lut.cpu())
+
+
+@pytest.mark.parametrize("u8", [False, True])
+@pytest.mark.parametrize("M,K,N", [(1, 5, 64), (63, 64, 65), (130, 67, 31), (2, 1, 70), (70, 129, 3)])
+def test_gemm2d_operands_contiguous_along_k(M, K, N, u8):
+    """Row and column operands contiguous along k (a linear layer's weight as
+    w.t()) around the 64 x 64 tiles of their packs, both orientations: the sums
+    and the u8 images against the int64 oracle."""
+    r = np.random.default_rng(M + K + N)
+    ai, bi = (r.integers(0, 256, s).astype(np.uint8) for s in ((M, K), (N, K)))
+    lut = r.integers(-32767, 32768, 65536)
+    lt = torch.from_numpy(lut.astype(np.float32)).cuda()
+    a, b = (torch.from_numpy(v if u8 else v.astype(np.float32)).cuda() for v in (ai, bi))
+    y, aq, bq = ops.gemm_fake_uint8_claude_save(a, b.t(), lt)
+    want = O.lut_gemm_i64(ai.T[None], bi, lut)[0].T
+    assert np.array_equal(y.cpu().numpy().astype(np.int64), want)
+    assert np.array_equal(aq.cpu().numpy(), ai) and np.array_equal(bq.cpu().numpy(), bi)
