@@ -151,7 +151,7 @@ __global__ void lut_prepare_kernel(const float* __restrict__ lut,
 // quad): the four taps' loads are in flight together and go out as four
 // 8-byte pieces.  Bound by HBM: 4 (fp32) or 1 byte read, 2 written per element
 // and 1 more for the fp32 operand's index image.  16 x 1152 x 784 fp32: 52 us
-// with one tap per thread, 27 us now (3.7 TB/s); the u8 operand 3.6 -> 6 TB/s.
+// with one tap per thread, 25 us now (4.0 TB/s); the u8 operand 3.6 -> 6 TB/s.
 template <typename T>
 __global__ void __launch_bounds__(256)
 pack_x_quads_kernel(const T* __restrict__ x, int N, int K, int L, int offset,
@@ -307,7 +307,7 @@ __global__ void pack_cols_strided_kernel(const T* __restrict__ y, int C, int K, 
 // The strided packs of operands contiguous along k (a linear layer's weight
 // [N, K], activations [M, K]): rows are far apart in memory, so lanes read along
 // k and a 64 x 64 tile of indices is turned in LDS; both sides then move whole
-// lines.  4096 x 1024 fp32: 34 -> 9 us; the columns of 1000 x 1024: 10.8 -> 5.
+// lines.  4096 x 1024 fp32: 34 -> 8.9 us; the columns of 1000 x 1024: 10.8 -> 5.5.
 constexpr int TT = 64;                 // tile side
 constexpr int TP = TT + 4;             // LDS bytes per tile row
 
