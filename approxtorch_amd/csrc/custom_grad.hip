@@ -70,7 +70,22 @@ struct Params {
   int tiles_r, tiles_o, nq; // nq = quads of taps
   int kq_chunk, kchunks;    // quads per workgroup, tap chunks
   int rchunk, rsteps;       // grad_w (resident tables): steps per workgroup, steps over R
+  int full;                 // leading workgroups on row tiles whose waves all have rows
 };
+
+// Workgroup order of the kernels with 2048-row tiles: contiguous ranges per
+// XCD over the full row tiles (neighbours share rows), then the last tile's
+// workgroups, if some of its waves have no rows, in dispatch order: a wave
+// without rows only builds its share of the tables, so these workgroups are
+// cheaper; dealt over all XCDs they fill the tail.  Rows 6272 (3.06 tiles):
+// grad_x of 128 x 1152 214 -> 172 us, grad_w of 512 x 2048 780 -> 748.
+__device__ __forceinline__ int tile_block(int full) {
+  const int bid = blockIdx.x;
+  if (bid >= full) return bid;
+  const int q = full >> 3, rem = full & 7;
+  const int xcd = bid & 7, slot = bid >> 3;
+  return xcd < rem ? xcd * (q + 1) + slot : rem * (q + 1) + (xcd - rem) * q + slot;
+}
 
 // DPP helpers (quad_perm / row_shr controls of the VOP DPP encoding).
 template <int CTRL>
@@ -265,7 +280,7 @@ custom_dx_kernel(const Params p) {
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
   const int rg = lane / 4, g = lane % 4;
-  const int lb = logical_block();
+  const int lb = tile_block(p.full);
   // A workgroup owns kq_chunk consecutive quads of taps of one row tile and
   // streams (quad, channel tile) steps through one table pipeline, so its
   // prologue is paid once per chunk, not once per quad.
@@ -405,8 +420,13 @@ custom_dx_kernel(const Params p) {
     load_dy<VEC>(dyr, dro, p.L, CT * tn, valid_of(tn), dyv);
   };
   auto quad_begin = [&](int) {};
-  table_stream(smem, p.tab, nsteps, col, rows, use, quad_end, quad_begin);
-  if constexpr (!MULTI) flush(j0);
+  if (tr * RT + __builtin_amdgcn_readfirstlane(wave) * RPW < p.R) {
+    table_stream(smem, p.tab, nsteps, col, rows, use, quad_end, quad_begin);
+    if constexpr (!MULTI) flush(j0);
+  } else {                                 // no rows: the wave's share of the tables
+    table_stream(smem, p.tab, nsteps, col, [](XRows&, int, int) {},
+                 [](auto, auto, int, const XRows&) {}, [](int) {}, [](int) {});
+  }
 }
 
 // ---------------------------------------- grad_w, tables rebuilt per row tile
@@ -427,7 +447,7 @@ custom_dw_tile_kernel(const Params p) {
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
   const int rg = lane / 4, g = lane % 4;
-  const int lb = logical_block();
+  const int lb = tile_block(p.full);
   const int to = lb % p.tiles_o;           // channel tile (consecutive blocks: same rows)
   const int kc = (lb / p.tiles_o) % p.kchunks;   // chunk of tap quads
   const int tr = lb / p.tiles_o / p.kchunks;     // row tile
@@ -537,7 +557,16 @@ custom_dw_tile_kernel(const Params p) {
     if (j >= 1) stage2(j - 1);
     if (j >= 2) stage3(j - 2);
   };
-  table_stream(smem, p.tab, nsteps, col, rows, use, quad_end, quad_begin);
+  if (tr * RT + __builtin_amdgcn_readfirstlane(wave) * RPW < p.R) {
+    table_stream(smem, p.tab, nsteps, col, rows, use, quad_end, quad_begin);
+  } else {                                 // no rows: tables and zero partial sums
+#pragma unroll
+    for (int s = 0; s < TPL; ++s)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[s][c] = 0.f;
+    table_stream(smem, p.tab, nsteps, col, [](XRows&, int, int) {},
+                 [](auto, auto, int, const XRows&) {}, quad_end, quad_begin);
+  }
   // drain the last two quads through stages 2 and 3
   if (nsteps >= 2) stage3(nsteps - 2);
   stage2(nsteps - 1);
@@ -998,6 +1027,9 @@ int lut_gemm_f32_tiled(const uint16_t* xt, int Rpad, const uint8_t* wt, int Opad
 
 }  // namespace atx
 
+// Row tiles of 2048 rows in which every wave has rows.
+static int full_row_tiles(int R) { return (int)cdiv(R - (cg::RT - cg::RPW), cg::RT); }
+
 extern "C" {
 
 int atx_custom_grad_dx(const uint16_t* xt, int Rpad, const uint8_t* wt, int Opad,
@@ -1029,6 +1061,7 @@ int atx_custom_grad_dx(const uint16_t* xt, int Rpad, const uint8_t* wt, int Opad
   }
   const long long blocks = (long long)p.tiles_r * p.kchunks;
   ATX_REQUIRE(blocks < 0x7fffffffLL, "atx_custom_grad_dx: grid too large");
+  p.full = full_row_tiles(p.R) * p.kchunks;
   const bool multi = p.kq_chunk > 1;
   if (L % 4 == 0 && multi)
     hipLaunchKernelGGL((cg::custom_dx_kernel<true, true>), dim3((unsigned)blocks), dim3(cg::NT),
@@ -1097,13 +1130,18 @@ static int custom_dw_run(const uint16_t* xt, int Rpad, const uint8_t* wt, int Op
     // workgroups to fill them (each workgroup writes its own taps' entries of
     // the row tile's slice, so no extra reduction).
     const long long tiles = (long long)p.tiles_r * p.tiles_o;
-    if (tiles < 256 && p.nq >= 16) {
-      const int want = (int)std::min<long long>(cdiv(256, tiles), p.nq / 8);
+    // With a last row tile that lacks rows for some waves, four times as many:
+    // its cheaper workgroups then fill the tail (3.06 row tiles x 32 channel
+    // tiles: 770 us with 256 or 512 workgroups, 748 with 1024, 769 with 2048).
+    const int target = full_row_tiles(p.R) < p.tiles_r ? 1024 : 256;
+    if (tiles < target && p.nq >= 16) {
+      const int want = (int)std::min<long long>(cdiv(target, tiles), p.nq / 8);
       p.kq_chunk = (int)cdiv(p.nq, want);
       p.kchunks = (int)cdiv(p.nq, p.kq_chunk);
     }
     const long long blocks = tiles * p.kchunks;
     ATX_REQUIRE(blocks < 0x7fffffffLL, "atx_custom_grad_dw: grid too large");
+    p.full = full_row_tiles(p.R) * p.tiles_o * p.kchunks;
     hipLaunchKernelGGL(cg::custom_dw_tile_kernel<false>, dim3((unsigned)blocks), dim3(cg::NT),
                        0, stream, p);
     rc = check_launch("custom_dw_tile_kernel");
