@@ -290,23 +290,6 @@ template <int B, bool VEC, bool SCALED> struct DataB {
   __device__ void advance() {}
 };
 
-// Implicit backward-data GEMM of a stride-1 conv (no col buffer, no fold):
-//   gx[n,c,h,w] = sum over p = t*O + o (t = i*KW + j) of
-//                 tx[wq[o][c*KK + t]] * go'[n, o, h + PH - i*DH, w + PW - j*DW]
-// (out-of-range go positions contribute 0).  With O % BK == 0 every k-tile
-// has one tap t, so its spatial shift is uniform over the tile.
-
-// Rows r = n*L + l of the weight GEMM's contraction, tracked incrementally:
-// the thread's quad starts at r = p0 + pq and moves by BK per k-tile.
-struct RowCursor {
-  int n, l;
-  __device__ void start(int r, int L) { n = r / L; l = r - n * L; }
-  __device__ void step(int d, int L) {
-    l += d;
-    while (l >= L) { l -= L; ++n; }
-  }
-};
-
 // Backward-weight A: A(m = o, p = r) = go[n][o][l] with r = n*L + l, read by
 // buffer loads from a descriptor that starts at image n0 (the image of the
 // block's first contraction row) and ends at the end of go: rows r >= P lie
