@@ -464,21 +464,26 @@ def conv_backward_data(go: Tensor, wq: Tensor, table: Tensor, g, mask=None, scal
     return img
 
 
-def gemm_backward_data(go: Tensor, wq: Tensor, table: Tensor) -> Tensor:
+def gemm_backward_data(go: Tensor, wq: Tensor, table: Tensor, bf16_table: bool = False) -> Tensor:
     """grad [N, K, L] of sum_k f(x, w) wrt x: sum_o go[n,o,l] * table[wq[o,k]] for
     go [N, O, L] and indices wq [O, K].
 
-    From 64 channels the split-bf16 GEMM (weight planes in a workspace) is the
-    more accurate and, from 256 channels or 4e8 products, the faster of the
-    two: 16 x 1152 x 784 x 128 41 us, error 1.8e-7 of the result against 53 us,
-    2.0e-7 of the fp32 matrix cores; 8 x 512 x 196 x 1024 32 us, 1.9e-7 against
-    93 us, 5.7e-7; 3 x 100 x 37 x 500 20 against 59 us.  Below, the fp32 kernels
-    (8 x 576 x 1000 x 33 1.0e-7 against 1.3e-7; 51 x 2776 x 19 x 17 10 against
-    14 us)."""
+    bf16_table: the caller knows that the table holds bf16 values (the
+    straight-through estimator's whole numbers).  The split-bf16 GEMM (weight
+    planes in a workspace) then forms exact products, and from 64 channels it
+    is the more accurate and, from 256 channels or 4e8 products, the faster of
+    the two: 4 x 576 x 784 x 128 error 1.2e-7 of the result against 2.0e-7 of
+    the fp32 matrix cores, 2 x 512 x 49 x 1024 1.3e-7 against 5.7e-7.
+
+    Any other table takes the fp32 kernels.  The split GEMM leaves out three
+    part products, which have the sign of the product: with operands of one
+    sign its result is short by 5e-8 of the sum of |terms| on average, whatever
+    the size (fp32: 1e-9 at 512 channels, 9e-9 at 4096), and an infinite go
+    times a zero part of a table value is NaN where the product is infinite."""
     goc = go.contiguous()
     N, O, Lc = goc.shape
     K = wq.size(1)
-    if O >= 64 and (O >= 256 or N * K * Lc * O >= 4e8) and \
+    if bf16_table and O >= 64 and (O >= 256 or N * K * Lc * O >= 4e8) and \
             6 * L.round_up(K, 128) * L.round_up(O, 32) < 2 ** 31:
         g = L.geom(N, K, 1, Lc, 1, 1, 1, 1, 0, 0, 1, 1)
         return conv_backward_data(goc, wq, table, g).view(N, K, Lc)

@@ -34,13 +34,14 @@ def _gemm_geom(N, K, L):
     return ops.L.geom(N, K, 1, L, 1, 1, 1, 1, 0, 0, 1, 1)
 
 
-def _gemm_grads(go, xq, wq, tx, tw):
-    """grad_x [N,K,L], grad_w [O,K] of sum_k f(x,w) with per-operand tables."""
+def _gemm_grads(go, xq, wq, tx, tw, bf16_table=False):
+    """grad_x [N,K,L], grad_w [O,K] of sum_k f(x,w) with per-operand tables
+    (bf16_table: tx holds bf16 values, as the decode tables do)."""
     N, K, L = xq.shape
     O = wq.size(0)
     g = _gemm_geom(N, K, L)
     go = go.contiguous()
-    col = ops.gemm_backward_data(go, wq, tx)
+    col = ops.gemm_backward_data(go, wq, tx, bf16_table)
     gw = ops.conv_backward_weight(go, xq.view(N, K, 1, L), tw, g, O, 128)
     return col, gw
 
@@ -62,7 +63,7 @@ class _bgemm_int8_ste(_bgemm_int8_base):
     def backward(ctx, grad_output):
         xq, wq = ctx.saved_tensors
         dec = decode_table(xq.device)
-        gx, gw = _gemm_grads(grad_output, xq, wq, dec, dec)
+        gx, gw = _gemm_grads(grad_output, xq, wq, dec, dec, bf16_table=True)
         return gx, gw, None
 
 

@@ -37,7 +37,7 @@ class _bgemm_uint8_ste(_bgemm_uint8_base):
     def backward(ctx, grad_output):
         xq, wq = ctx.saved_tensors
         ident = decode_table(xq.device, signed=False)
-        gx, gw = _gemm_grads(grad_output, xq, wq, ident, ident)
+        gx, gw = _gemm_grads(grad_output, xq, wq, ident, ident, bf16_table=True)
         return gx, gw, None
 
 
