@@ -1121,16 +1121,42 @@ __device__ __forceinline__ void mma_stage(const char* st, floatx4 (&part)[2][4])
   }
 }
 
+// acc += a tap's sums in the columns whose output the tap reads.  With a
+// non-finite entry in the table, the zeros that stand for outputs outside go
+// give products of NaN, and the tap adds nothing there (nor does it with a
+// finite table, where the products are zero).
+template <bool TR>
+__device__ __forceinline__ void add_reached(floatx4 (&acc)[2][4], const floatx4 (&part)[2][4],
+                                            const TapArgs& p, const TapClass& k, int n0,
+                                            int tap) {
+  const int a = tap / k.nJ, b = tap - a * k.nJ, HWc = k.Hc * k.Wc;
+  const int dh = k.dh0 - a * k.dhs, dw = k.dw0 - b * k.dws;
+  const int lane = threadIdx.x & 63;
+  const int c0 = n0 + ((threadIdx.x >> 6) & 1) * 64 + (TR ? 4 * (lane >> 4) : lane & 15);
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {            // TR: the block's columns; else its rows
+      const int q = (c0 + 16 * j + (TR ? e : 0)) % HWc, hc = q / k.Wc, wc = q - hc * k.Wc;
+      const bool in = (unsigned)(hc + dh) < (unsigned)p.g.OH &&
+                      (unsigned)(wc + dw) < (unsigned)p.g.OW;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        acc[i][j][e] = in ? acc[i][j][e] + part[i][j][e] : acc[i][j][e];
+    }
+}
+
 // acc += the products of `tiles` k-tiles.  A tap's sum, or at most FLUSH
 // k-tiles of it, is accumulated on its own and then added: one chain over all
 // taps and channels doubled the error of 9 x 128 terms against per-tap sums
 // (5.2e-7 against 2.0e-7 of the result).
 constexpr int FLUSH = 2;
-template <int BM, bool EXACT, bool TR>
+template <int BM, bool EXACT, bool TR, bool FINITE>
 __device__ __forceinline__ void tap_sums(TapLoader<BM>& ld, const TapArgs& p, const TapClass& k,
-                                         int tiles, floatx4 (&acc)[2][4], char* st0, char* st1) {
+                                         int n0, int tiles, floatx4 (&acc)[2][4], char* st0,
+                                         char* st1) {
   floatx4 part[2][4];
-  int run = 0, ob = ld.ob;
+  int run = 0, ob = ld.ob, tap = ld.a * k.nJ + ld.b;
   ld.load(p, k, st0);
   auto step = [&](char* cur, char* nxt, int left) __attribute__((always_inline)) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's copies are in LDS
@@ -1146,10 +1172,15 @@ __device__ __forceinline__ void tap_sums(TapLoader<BM>& ld, const TapArgs& p, co
     if (++ob == p.nOb) ob = 0;
     if (++run == FLUSH || ob == 0 || left == 1) {
       run = 0;
+      if constexpr (FINITE) {
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] += part[i][j];
+          for (int j = 0; j < 4; ++j) acc[i][j] += part[i][j];
+      } else {
+        add_reached<TR>(acc, part, p, k, n0, tap);
+      }
+      if (ob == 0) ++tap;
     }
   };
   for (; tiles > 1; tiles -= 2) {
@@ -1180,12 +1211,22 @@ tap_planes_kernel(const TapArgs p, DataOut ep, const float* __restrict__ tx) {
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-  const bool exact = __syncthreads_or(t < 256 && bf16_rest(tx[t & 255]) != 0.0f) == 0;
+  bool rest = false, wild = false;         // each wave reads the whole table: no barrier
+#pragma unroll
+  for (int e = 0; e < 256; e += 64) {
+    const float v = tx[e + (t & 63)];
+    rest |= bf16_rest(v) != 0.0f;
+    wild |= !__builtin_isfinite(v);
+  }
+  const bool exact = !__any(rest), finite = !__any(wild);
   if (tb < te) {
     TapLoader<BM> ld;
     ld.init(p, k, m0, n0, cols, tb, !exact);
-    if (exact) tap_sums<BM, true, VO>(ld, p, k, te - tb, acc, st0, st1);
-    else tap_sums<BM, false, VO>(ld, p, k, te - tb, acc, st0, st1);
+    const int n = te - tb;
+    if (exact && finite) tap_sums<BM, true, VO, true>(ld, p, k, n0, n, acc, st0, st1);
+    else if (finite) tap_sums<BM, false, VO, true>(ld, p, k, n0, n, acc, st0, st1);
+    else if (exact) tap_sums<BM, true, VO, false>(ld, p, k, n0, n, acc, st0, st1);
+    else tap_sums<BM, false, VO, false>(ld, p, k, n0, n, acc, st0, st1);
   }
   // epilogue, with the fused STE (mask ? v : 0) / max(scale, 1e-12)
   const int lane = t & 63, wave = t >> 6;

@@ -18,6 +18,17 @@ from approxtorch_amd.backend import ops
 pytestmark = pytest.mark.gpu
 
 
+def uses_tap_gemm(g, Oc):
+    """Whether atx_conv_bwd_data takes the tap GEMM: its workspace holds the
+    weight planes, the go planes and whole partial images, and not columns."""
+    K, P = g.C * g.KH * g.KW, g.N * g.OH * g.OW
+    rest = L.query("atx_conv_bwd_data_workspace_bytes", g, Oc) - \
+        6 * L.round_up(K, 128) * L.round_up(Oc, 32) - \
+        L.round_up(P * 6 * L.round_up(Oc, 32), 256)
+    image = 4 * g.N * g.C * g.H * g.W
+    return rest % image == 0 and rest // image in (0, *range(2, 65))
+
+
 def check(N, C, H, W, Oc, k, s, p, d, table, fused, seed=0):
     gen = torch.Generator(device="cuda").manual_seed(seed)
     g = ops.conv_geom((N, C, H, W), k, s, p, d)
@@ -63,3 +74,34 @@ def test_tap_gemm_two_passes():
     g = ops.conv_geom((13, 1, 1024, 1024), 3, 1, 1, 1)
     assert L.query("atx_conv_bwd_data_workspace_bytes", g, 2) < 2 ** 31 + 2 ** 20
     check(13, 1, 1024, 1024, 2, 3, 1, 1, 1, "general", True)
+
+
+@pytest.mark.parametrize("table", ["exact", "general"])
+@pytest.mark.parametrize("N,C,H,W,Oc,k,s,p,d", [
+    (8, 64, 28, 28, 64, 3, 1, 1, 1), (8, 70, 33, 31, 65, 3, 1, 1, 1), (16, 66, 35, 31, 72, 3, 2, 1, 1),
+    (16, 130, 34, 30, 64, 3, 2, 2, 2), (16, 72, 40, 38, 64, (2, 3), 2, 0, 1)])
+def test_non_finite_table_entries_stay_with_their_taps(N, C, H, W, Oc, k, s, p, d, table):
+    """A tap adds nothing to the pixels whose output lies outside go, also when
+    its factor is infinite or NaN: everything else keeps its finite value."""
+    gen = torch.Generator(device="cuda").manual_seed(C)
+    g = ops.conv_geom((N, C, H, W), k, s, p, d)
+    go = torch.randn(N, Oc, g.OH, g.OW, generator=gen, device="cuda")
+    wq = torch.randint(2, 256, (Oc, C, g.KH, g.KW), generator=gen, device="cuda",
+                       dtype=torch.uint8)
+    wq[1, ::2, 0, 0], wq[Oc - 1, 1::3, g.KH - 1, g.KW - 1] = 0, 1
+    wq = wq.view(Oc, -1)
+    tx = torch.arange(256, device="cuda").float() if table == "exact" else \
+        torch.randn(256, generator=gen, device="cuda")
+    tx[0], tx[1] = float("inf"), float("nan")
+    assert uses_tap_gemm(g, Oc)
+    gx = ops.conv_backward_data(go, wq, tx, g)
+    wt = tx[wq.long()].double().t().contiguous()
+    for n in range(N):
+        v = go[n].double().reshape(Oc, -1)
+        want, terms = (F.fold((a @ b).unsqueeze(0), (H, W), (g.KH, g.KW), d, p, s)[0]
+                       for a, b in ((wt, v), (wt.abs(), v.abs())))
+        ok = torch.isfinite(want)
+        assert torch.equal(torch.isfinite(gx[n]), ok)
+        assert bool(((gx[n].double() - want).abs()[ok] <= 1e-5 * terms[ok] + 1e-6).all())
+        if p or s == 1:
+            assert bool(ok[::2].any()) and not bool(ok.all())
