@@ -577,9 +577,10 @@ static DwRuns dw_runs(const atx_conv_geom& g) {
 
 // 3x3 kernels with a square stride of 1 or 2 and a square dilation of 1 or 2
 // (every other geometry takes the general kernels), sizes within the strip
-// kernels' 32-bit counts.
+// kernels' 32-bit counts.  An empty image (all of it padding) has no row or
+// column that the strips' clamped loads could read.
 static bool dw_strips(const atx_conv_geom& g) {
-  return g.OH > 0 && g.OW > 0 && g.KH == 3 && g.KW == 3 && g.SH == g.SW &&
+  return g.H > 0 && g.W > 0 && g.OH > 0 && g.OW > 0 && g.KH == 3 && g.KW == 3 && g.SH == g.SW &&
          (g.SW == 1 || g.SW == 2) && g.DH == g.DW && (g.DW == 1 || g.DW == 2) &&
          (long long)g.N * g.H * ((g.W + 3) / 4) < (1LL << 30) &&
          (long long)g.N * g.OH * ((g.OW + 3) / 4) < (1LL << 30);

@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 import torch
 
+from approxtorch_amd.backend import _lib as L
 from approxtorch_amd.backend import ops
 
 pytestmark = pytest.mark.gpu
@@ -80,3 +81,20 @@ def test_strip_gradients_keep_non_finite_table_entries_to_their_taps():
     gx = ops.dwconv_backward_data(torch.ones(1, 1, 6, 6, device="cuda"), wq, tx, g)[0, 0]
     assert torch.isinf(gx[:5, :5]).all()
     assert (gx[5] == 0).all() and (gx[:, 5] == 0).all()
+
+
+@pytest.mark.parametrize("H,W", [(0, 4), (4, 0), (0, 0)])
+def test_weight_gradient_of_an_empty_image(H, W):
+    """An image without rows or columns is all padding: no load of it, and every
+    tap's gradient is the sum of go times the padding's factor."""
+    g = ops.conv_geom((2, 3, H, W), 3, 1, 2, 1)
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    go = torch.randn(2, 3, g.OH, g.OW, generator=gen, device="cuda")
+    img = torch.zeros(64, dtype=torch.int8, device="cuda")      # a valid pointer to no pixels
+    tw = torch.randn(256, generator=gen, device="cuda")
+    ws = torch.empty(L.query("atx_dwconv_bwd_weight_workspace_bytes", g) // 4, device="cuda")
+    gw = torch.empty(3, 9, device="cuda")
+    L.call("atx_dwconv_bwd_weight", L.ptr(go), L.ptr(img), 0, g, 77, None, L.ptr(tw), None, None,
+           None, None, L.ptr(gw), L.ptr(ws), L.stream_of(go))
+    want = (go * tw[77]).double().sum((0, 2, 3)).unsqueeze(1).expand(3, 9)
+    assert bool(((gw.double() - want).abs() <= 1e-5).all())
