@@ -98,3 +98,19 @@ def test_weight_gradient_of_an_empty_image(H, W):
            None, None, L.ptr(gw), L.ptr(ws), L.stream_of(go))
     want = (go * tw[77]).double().sum((0, 2, 3)).unsqueeze(1).expand(3, 9)
     assert bool(((gw.double() - want).abs() <= 1e-5).all())
+
+
+def test_weight_gradient_of_a_long_batch():
+    """15360 images of 1 x 4 over 2048 channels: one 1 in each of the first 256
+    images, 2^-24 (half an ulp of 1, which a chain beside it drops) elsewhere.
+    Chains of at most two tasks lose at most 8 x 2^-24 of the result beside
+    the 1s, and 32 partial sums as many roundings: 2e-6 bounds both; one
+    chain over the batch would lose 1.4e-5."""
+    N, C = 15360, 2048
+    g = ops.conv_geom((N, C, 1, 4), 3, 1, 1, 1)
+    go = torch.full((N, C, 1, 4), 2.0 ** -24, device="cuda")
+    go[:256, :, 0, 0] = 1.0
+    img = torch.zeros(N, C, 1, 4, dtype=torch.int8, device="cuda")
+    gw = ops.dwconv_backward_weight(go, img, torch.ones(256, device="cuda"), g, 128)
+    want = 256 + (N * 4 - 256) * 2.0 ** -24
+    assert float((gw.double() / want - 1).abs().max()) <= 2e-6
