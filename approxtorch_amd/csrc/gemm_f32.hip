@@ -530,7 +530,9 @@ template <int B> struct PlaneA {
 template <int B, bool VEC, bool SCALED> struct GoCols {
   static_assert(B == 128, "GoCols covers 128 columns with 256 threads");
   __amdgpu_buffer_rsrc_t res;
-  int O, L;
+  int O, L;                 // L: positions of go per image
+  int Lc;                   // columns per image
+  int W, OW, first;         // W > 0: column q is go's position (q / W) * OW + q % W + first
   const float* sx; const float* sw;
   int oq, cq;
   unsigned off[4];          // byte offset of column 4cq + e at o = 0 (VEC: off[0] only)
@@ -538,15 +540,17 @@ template <int B, bool VEC, bool SCALED> struct GoCols {
   float sc[4];
   __device__ void init(const float* go, long long go_elems, int tid, int n0, int NL) {
     oq = tid & 7; cq = tid >> 3;
-    const int nb = n0 / L;
+    const int nb = n0 / Lc;
     const long long base = (long long)nb * O * L;
     const long long bytes = (go_elems - base) * 4;
     res = buffer_rsrc(go + base, (int)(bytes < 0x7fffffffLL ? bytes : 0x7fffffffLL));
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int c = n0 + 4 * cq + e;
-      const int n = c / L;
-      off[e] = c < NL ? (unsigned)(((long long)(n - nb) * O * L + (c - n * L)) * 4) : 0x80000000u;
+      const int n = c / Lc;
+      int l = c - n * Lc;
+      if (!VEC && W > 0) l = l / W * OW + l % W + first;
+      off[e] = c < NL ? (unsigned)(((long long)(n - nb) * O * L + l) * 4) : 0x80000000u;
     }
   }
   __device__ void fetch(int p0, int) {
@@ -1414,6 +1418,10 @@ struct DataArgs {
   int splits, o_chunk;                       // contraction split (1 = none)
   float* partials;                           // [splits][N*K*L] when splits > 1
   uint16_t* planes;                          // bf16 weight planes (null: fp32 kernels)
+  // A padded 1x1 conv (or null; with planes): only go's positions inside the
+  // image are columns, and out is the image gradient.
+  const atx_conv_geom* crop = nullptr;
+  int columns() const { return crop ? crop->H * crop->W : L; }   // per image
 };
 
 // Bytes of the bf16 weight planes [3][Kp][Opad] (Kp = K rounded up to 128,
@@ -1478,14 +1486,18 @@ static void launch_data(const DataArgs& a, hipStream_t stream) {
 
 template <int BM, bool VB, bool SC>
 static void launch_data_planes(const DataArgs& a, hipStream_t stream) {
-  const int NL = a.N * a.L;
+  const int Lc = a.columns(), NL = a.N * Lc;
   PlaneA<BM> la{};
   la.planes = a.planes; la.pbytes = (int)weight_planes_bytes(a.K, a.O);
   la.Kp = (int)(cdiv(a.K, 128) * 128); la.Opad = (int)(cdiv(a.O, BK) * BK);
   GoCols<128, VB, SC> lb{};
-  lb.O = a.O; lb.L = a.L; lb.sx = a.sx; lb.sw = a.sw;
+  lb.O = a.O; lb.L = a.L; lb.Lc = Lc; lb.sx = a.sx; lb.sw = a.sw;
+  if (a.crop) {
+    lb.W = a.crop->W; lb.OW = a.crop->OW;
+    lb.first = a.crop->PH * a.crop->OW + a.crop->PW;
+  }
   const bool split = a.splits > 1;
-  DataOut ep{split ? a.partials : a.out, a.K, a.L, NL, split ? nullptr : a.mask,
+  DataOut ep{split ? a.partials : a.out, a.K, Lc, NL, split ? nullptr : a.mask,
              split ? nullptr : a.scale, (long long)NL * a.K};
   dim3 grid((unsigned)cdiv(NL, 128), (unsigned)cdiv(a.K, BM), (unsigned)a.splits);
   hipLaunchKernelGGL((data_planes_kernel<BM, VB, SC>), grid, dim3(GT), 0, stream, la, lb, ep,
@@ -1496,7 +1508,8 @@ template <int BM, bool SC>
 static void dispatch_data_vec(const DataArgs& a, hipStream_t stream) {
   const bool va = a.K % 4 == 0 && (uintptr_t)a.wq % 4 == 0;
   const float* out = a.splits > 1 ? a.partials : a.out;
-  const bool vb = a.L % 4 == 0 && (uintptr_t)a.go % 16 == 0 && (uintptr_t)out % 16 == 0 &&
+  const bool vb = !a.crop && a.L % 4 == 0 && (uintptr_t)a.go % 16 == 0 &&
+                  (uintptr_t)out % 16 == 0 &&
                   (a.splits > 1 || (uintptr_t)a.mask % 4 == 0);
   if (a.planes) {
     if (vb) launch_data_planes<BM, true, SC>(a, stream);
@@ -1516,7 +1529,7 @@ static int run_data_gemm(DataArgs a, hipStream_t stream) {
   if (a.splits < 1) a.splits = 1;
   a.o_chunk = (int)(cdiv(cdiv(a.O, a.splits), BK) * BK);
   a.splits = (int)cdiv(a.O, a.o_chunk);
-  if (a.planes && !planes_fit(a.L, a.O, a.L)) a.planes = nullptr;
+  if (a.planes && !planes_fit(a.columns(), a.O, a.L)) a.planes = nullptr;
   if (a.planes) {
     const int rc = launch_weight_planes(a.wq, a.tx, a.O, a.K, a.planes, stream);
     if (rc) return rc;
@@ -1529,7 +1542,7 @@ static int run_data_gemm(DataArgs a, hipStream_t stream) {
   }
   int rc = check_launch("data_gemm_kernel");
   if (rc || a.splits == 1) return rc;
-  const long long numel = (long long)a.N * a.K * a.L;
+  const long long numel = (long long)a.N * a.K * a.columns();
   // split_sum's per-channel scale index i / K: K = numel makes it per tensor
   return launch_split_sum(a.partials, a.splits, numel, (int)numel, a.mask, a.scale, a.out,
                           stream);
@@ -1801,8 +1814,17 @@ static bool direct_columns(const atx_conv_geom& g) {
   return g.KH == 1 && g.KW == 1 && g.SH == 1 && g.SW == 1 && g.PH == 0 && g.PW == 0;
 }
 
+// A padded 1x1, stride-1 conv's columns inside the image are its gradient: the
+// GEMM reads go's positions there (scalar loads).  Against columns and col2im,
+// 64 x 64 x 56 x 56 -> 64 with padding 1: 65 -> 43 us, 64 x 256 x 28 x 28 ->
+// 256: 97 -> 78.
+static bool cropped_columns(const atx_conv_geom& g, int O) {
+  return g.KH == 1 && g.KW == 1 && g.SH == 1 && g.SW == 1 && !direct_columns(g) && g.H > 0 &&
+         g.W > 0 && planes_fit((long long)g.H * g.W, O, (long long)g.OH * g.OW);
+}
+
 // Workspace of atx_conv_bwd_data: [bf16 weight planes][split partials][col
-// (unless direct)], or the tap GEMM's (tap_workspace_bytes).
+// (unless direct or cropped)], or the tap GEMM's (tap_workspace_bytes).
 long long atx_conv_bwd_data_workspace_bytes(atx_conv_geom g, int O) {
   const int K = g.C * g.KH * g.KW, L = g.OH * g.OW;
   if (g.N <= 0 || K <= 0 || L <= 0 || O <= 0) return 0;
@@ -1817,9 +1839,11 @@ long long atx_conv_bwd_data_workspace_bytes(atx_conv_geom g, int O) {
     }
     return bytes;
   }
-  const long long numel = (long long)g.N * K * L;
-  const int S = data_splits(g.N, O, K, L);
-  return planes + ((S > 1 ? S : 0) + (direct_columns(g) ? 0 : 1)) * numel * 4;
+  const bool crop = cropped_columns(g, O);
+  const int Lc = crop ? g.H * g.W : L;
+  const long long numel = (long long)g.N * K * Lc;
+  const int S = data_splits(g.N, O, K, Lc);
+  return planes + ((S > 1 ? S : 0) + (crop || direct_columns(g) ? 0 : 1)) * numel * 4;
 }
 
 int atx_conv_bwd_data(const float* go, const uint8_t* wq, const float* tx, atx_conv_geom g,
@@ -1847,19 +1871,21 @@ int atx_conv_bwd_data(const float* go, const uint8_t* wq, const float* tx, atx_c
     ATX_REQUIRE(go && wq && tx, "atx_conv_bwd_data: null pointer");
     return run_tap_gemm(go, wq, tx, g, O, go_sx, go_sw, mask, scale, gx, (char*)workspace, stream);
   }
-  const long long numel = (long long)g.N * K * L;
-  const int S = (O > 0 && numel > 0) ? data_splits(g.N, O, K, L) : 1;
+  const bool crop = O > 0 && L > 0 && cropped_columns(g, O);
+  const int Lc = crop ? g.H * g.W : L;
+  const long long numel = (long long)g.N * K * Lc;
+  const int S = (O > 0 && numel > 0) ? data_splits(g.N, O, K, Lc) : 1;
   float* partials = S > 1 ? rest : nullptr;
   float* col = rest ? rest + (S > 1 ? S * numel : 0) : nullptr;
   ATX_REQUIRE(S == 1 || rest, "atx_conv_bwd_data: null workspace");
-  if (direct_columns(g)) {
+  if (crop || direct_columns(g)) {
     if (O == 0 || L == 0)
       return launch_split_sum(nullptr, 0, img, 1, nullptr, nullptr, gx, stream);
     ATX_REQUIRE(go && wq && tx, "atx_conv_bwd_data: null pointer");
     ATX_REQUIRE((long long)g.N * L < 0x7fffffffLL && cdiv(K, 64) <= 65535,
                 "atx_conv_bwd_data: sizes too large");
     const DataArgs a{go, wq, tx, g.N, O, K, L, go_sx, go_sw, gx, mask, scale, S, 0, partials,
-                     planes};
+                     planes, crop ? &g : nullptr};
     return run_data_gemm(a, stream);
   }
   ATX_REQUIRE(rest, "atx_conv_bwd_data: null workspace");

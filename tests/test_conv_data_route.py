@@ -1,0 +1,29 @@
+"""Which way atx_conv_bwd_data goes to an image gradient, told from its
+workspace (a host query, no GPU): no columns for a padded 1x1 conv."""
+import pytest
+
+from approxtorch_amd.backend import _lib as L
+from approxtorch_amd.backend import ops
+
+
+def route(shape, Oc, k, s, p, d=1):
+    g = ops.conv_geom(shape, k, s, p, d)
+    K, P = g.C * g.KH * g.KW, g.N * g.OH * g.OW
+    rest = L.query("atx_conv_bwd_data_workspace_bytes", g, Oc) - \
+        6 * L.round_up(K, 128) * L.round_up(Oc, 32)
+    planes = L.round_up(P * 6 * L.round_up(Oc, 32), 256)
+    image, columns = 4 * g.N * g.C * g.H * g.W, 4 * K * P
+    slices = (0, *range(2, 65))
+    # stride 1: the columns are KH KW images, so they are looked for first
+    return next(name for name, ok in (
+        ("tap", (rest - planes) % image == 0 and (rest - planes) // image in slices),
+        ("columns", rest % columns == 0 and rest // columns - 1 in slices),
+        ("image", rest % image == 0 and rest // image in slices)) if ok)
+
+
+@pytest.mark.parametrize("shape,Oc,k,s,p,way", [
+    ((64, 64, 56, 56), 64, 1, 1, 1, "image"),
+    ((2, 24, 9, 11), 40, 1, 1, (0, 2), "image"),
+    ((64, 64, 56, 56), 64, 1, 1, 0, "image")])
+def test_route(shape, Oc, k, s, p, way):
+    assert route(shape, Oc, k, s, p) == way

@@ -76,6 +76,22 @@ def test_tap_gemm_two_passes():
     check(13, 1, 1024, 1024, 2, 3, 1, 1, 1, "general", True)
 
 
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("table", ["exact", "general"])
+@pytest.mark.parametrize("N,C,H,W,Oc,p", [
+    (3, 33, 9, 11, 40, 1), (2, 130, 12, 8, 96, (0, 2)), (5, 64, 1, 1, 33, 3), (2, 24, 7, 7, 520, 1),
+    (16, 64, 56, 56, 64, 1)])
+def test_padded_1x1(N, C, H, W, Oc, p, table, fused):
+    """The image gradient of a padded 1x1 conv from go's positions inside the
+    image, without columns: ragged sizes, paddings of either axis, a split
+    contraction."""
+    g = ops.conv_geom((N, C, H, W), 1, 1, p, 1)
+    rest = L.query("atx_conv_bwd_data_workspace_bytes", g, Oc) - \
+        6 * L.round_up(C, 128) * L.round_up(Oc, 32)
+    assert rest % (4 * N * C * H * W) == 0
+    check(N, C, H, W, Oc, 1, 1, p, 1, table, fused)
+
+
 @pytest.mark.parametrize("table", ["exact", "general"])
 @pytest.mark.parametrize("N,C,H,W,Oc,k,s,p,d", [
     (8, 64, 28, 28, 64, 3, 1, 1, 1), (8, 70, 33, 31, 65, 3, 1, 1, 1), (16, 66, 35, 31, 72, 3, 2, 1, 1),
