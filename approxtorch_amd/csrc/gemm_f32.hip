@@ -33,6 +33,7 @@
 #include "atx_tiles.h"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace atx {
@@ -1696,25 +1697,81 @@ static bool tap_size(const atx_conv_geom& g, int O) {
          (g.SH == 1 && g.SW == 1 && (double)g.N * g.H * g.W * cdiv(g.C, 64) >= 512 * 128);
 }
 
+// Times of the two ways to an image gradient in microseconds, least-squares
+// fits to 220 convs (the 3x3 layers of the ResNets, small C or O, and random
+// ones: kernels of 2 to 7, strides 1 and 2, dilations, C and O from 1 to 512),
+// each with a bf16-exact and a general table; they are off by 14% and 13% (rms).
+// Both count the padding they multiply.
+//
+// The tap GEMM pads C to a tile of 64 or 128 rows for each tap and go to 32
+// channels: k-tile rounds (64 rows: two blocks per CU, 128: one), blocks, the
+// planes (4 bytes read, 6 written and 6 read per value), gx with its mask and
+// partials, and stride 2's scattered stores.
+static double tap_cost(const atx_conv_geom& g, int O) {
+  const TapClasses t = tap_classes(g);
+  const double P = (double)g.N * g.OH * g.OW, img = (double)g.N * g.C * g.H * g.W;
+  const long long nob = cdiv(O, BK), S = tap_splits(g, O);
+  const long long slots = g.C <= 64 ? 512 : 256, mt = cdiv(g.C, g.C <= 64 ? 64 : 128);
+  double blocks = 0.0, work = 0.0;
+  for (int i = 0; i < t.n; ++i) {
+    const double b = (double)cdiv((long long)g.N * t.c[i].Hc * t.c[i].Wc, 128) * mt;
+    blocks += b;
+    work += b * t.c[i].nI * t.c[i].nJ * nob / slots;
+  }
+  const double chain = (double)cdiv((long long)t.c[0].nI * t.c[0].nJ * nob, S);
+  const double rounds = t.n == 1 ? std::ceil(blocks * S / slots) : 1.0;
+  return 15.6 + 0.92 * std::max(work, chain * rounds) + 2.9 * blocks * S / slots +
+         0.31e-6 * P * (4.0 * O + 192.0 * nob) + 0.18e-6 * img * (5.0 + (S > 1 ? 8.0 * S : 0.0)) +
+         (t.n > 1 ? 3.2e-6 * img : 0.0);
+}
+
+// Share of a tile's rows and channels that are not padding.
+static double tap_fill(const atx_conv_geom& g, int O) {
+  const double tile = g.C <= 64 ? 64.0 : 128.0;
+  return g.C / (std::ceil(g.C / tile) * tile) * O / (cdiv(O, BK) * (double)BK);
+}
+
+// The column GEMM pads C KH KW to its row tile (64 or 128) and O to 32; then
+// the columns, written and folded (more per pixel with stride 2).
+static double column_cost(const atx_conv_geom& g, int O) {
+  const int K = g.C * g.KH * g.KW, L = g.OH * g.OW;
+  const double P = (double)g.N * L, img = (double)g.N * g.C * g.H * g.W;
+  const long long S = data_splits(g.N, O, K, L), nob = cdiv(O, BK);
+  const double tile = tile_of(K) / 64.0;
+  const double blocks = (double)cdiv((long long)g.N * L, 128) * cdiv(K, tile_of(K));
+  return 13.7 + 0.42 * std::ceil(blocks * S / 512.0) * (cdiv(nob, S) + 4.0) * tile +
+         0.79 * blocks * nob * tile / 512.0 + 0.04e-6 * P * O * 4.0 +
+         0.22e-6 * (P * K * (4.0 + (S > 1 ? 8.0 * S : 0.0)) + 5.0 * img) +
+         0.19e-6 * img * g.KH * g.KW + (g.SH > 1 || g.SW > 1 ? 1.0e-6 * img : 0.0);
+}
+
 // The tap GEMM serves convs of at least two taps, strides of 1 or 2 and
-// tap_size().  A 1x1 conv's columns are its gradient, or (stride 2) most of its
-// pixels have no tap: the column GEMM there reads go once per 128 rows and
-// writes the result, which the go planes' pass does not beat (1024 -> 256 at
-// 14 x 14, batch 64: 74 against 85 us).  Below 1e8 products the extra launch
-// costs more than the loop saves (1.8e6 to 5.5e6 products: 14-18 us against
-// 17-19; 3e8: 27.5 against 24.6).  Above, on the 3x3 layers of ResNet-50 at
-// batch 64 and ResNet-18 at 128 with LRE tables, against the column GEMM plus
-// col2im or the implicit GEMM that read go itself: 56 x 56 x 64 186 -> 140 us,
-// 28 x 28 x 128 191 -> 130, 14 x 14 x 256 144 -> 133, 7 x 7 x 512 143 -> 122,
-// stride 2 at 56 x 56 x 128 256 -> 206, 16 x 16 x 128 126 -> 79; with a
-// bf16-exact (STE) table 159 -> 89 and 106 -> 54 at 28 x 28 and 16 x 16.
+// tap_size() where the estimates above favour it; with tiles filled to 90%
+// also where it is estimated up to 1.2 times as long, about the estimates'
+// error, since it is the faster there more often (128 -> 256 with stride 2 at
+// 16 x 16, batch 128: 66 against 77 us, both estimated 72).  A 1x1 conv's
+// columns are its gradient, or (stride 2) most of its pixels have no tap: the
+// column GEMM there reads go once per 128 rows and writes the result, which
+// the go planes' pass does not beat (1024 -> 256 at 14 x 14, batch 64: 74
+// against 85 us).  Below 1e8 products the extra launch costs more than the
+// loop saves (1.8e6 to 5.5e6 products: 14-18 us against 17-19; 3e8: 27.5
+// against 24.6).  Above, LRE tables, tap GEMM against column GEMM plus col2im:
+// batch 64 at 56 x 56 x 64 137 / 296 us, 28 x 28 x 128 126 / 175, 14 x 14 x 256
+// 129 / 139, 7 x 7 x 512 119 / 135, stride 2 at 56 x 56 x 128 205 / 242; few
+// output channels (64 -> 8 at 56 x 56) 82 / 248.  The columns win where padding
+// is most of the tap GEMM's work: 3 -> 64 at 64 x 64 125 / 38, 4 -> 512 1337 /
+// 172, 7x7 stride 2 of 3 -> 64 at 224 x 224, batch 32 803 / 241, 24 -> 24 with
+// stride 2 66 / 48.  Over 220 further random convs with both tables the tap
+// GEMM wherever tap_size() holds takes 50.6 ms, the faster way of each 31.0
+// and the rule's picks 31.7.
 static bool tap_gemm(const atx_conv_geom& g, int O) {
   const long long K = (long long)g.C * g.KH * g.KW, L = (long long)g.OH * g.OW;
   return g.KH * g.KW > 1 && (g.SH == 1 || g.SH == 2) && (g.SW == 1 || g.SW == 2) && O > 0 &&
          g.N > 0 && K > 0 && L > 0 && g.H > 0 && g.W > 0 &&
          tap_size(g, O) && weight_planes_bytes((int)K, O) < 0x7fffffffLL &&
          (double)g.KH * g.KW * cdiv(O, BK) < 1e8 && cdiv(g.C, 64) <= 65535 &&
-         cdiv(O, BK) <= 65535 && tap_images(g, O) > 0;
+         cdiv(O, BK) <= 65535 && tap_images(g, O) > 0 &&
+         tap_cost(g, O) < column_cost(g, O) * (tap_fill(g, O) >= 0.9 ? 1.2 : 1.0);
 }
 
 // Workspace of one pass: [weight planes][go planes][split partials].

@@ -1,5 +1,7 @@
 """Which way atx_conv_bwd_data goes to an image gradient, told from its
-workspace (a host query, no GPU): no columns for a padded 1x1 conv."""
+workspace (a host query, no GPU): the tap GEMM where it measured faster, the
+columns where padding would be most of its work, and no columns for a padded
+1x1 conv."""
 import pytest
 
 from approxtorch_amd.backend import _lib as L
@@ -21,7 +23,21 @@ def route(shape, Oc, k, s, p, d=1):
         ("image", rest % image == 0 and rest // image in slices)) if ok)
 
 
+# (tap GEMM, columns and their fold in us, LRE table)
 @pytest.mark.parametrize("shape,Oc,k,s,p,way", [
+    ((64, 64, 56, 56), 64, 3, 1, 1, "tap"),             # 137 / 296
+    ((64, 128, 28, 28), 128, 3, 1, 1, "tap"),           # 126 / 175
+    ((64, 512, 7, 7), 512, 3, 1, 1, "tap"),             # 119 / 135
+    ((64, 128, 56, 56), 128, 3, 2, 1, "tap"),           # 205 / 242
+    ((64, 64, 56, 56), 8, 3, 1, 1, "tap"),              # 82 / 248
+    ((128, 256, 28, 28), 8, 3, 1, 1, "tap"),            # 147 / 466
+    ((64, 3, 64, 64), 64, 3, 1, 1, "columns"),          # 125 / 38
+    ((64, 8, 56, 56), 128, 3, 1, 1, "columns"),         # 270 / 77
+    ((64, 4, 64, 64), 512, 3, 1, 1, "columns"),         # 1337 / 172
+    ((32, 3, 224, 224), 64, 7, 2, 3, "columns"),        # 803 / 241
+    ((64, 24, 56, 56), 24, 3, 2, 1, "columns"),         # 66 / 48
+    ((13, 1, 1024, 1024), 2, 3, 1, 1, "columns"),       # 3262 / 693
+    ((76, 3, 24, 126), 131, 3, 1, 1, "columns"),        # 366 / 59
     ((64, 64, 56, 56), 64, 1, 1, 1, "image"),
     ((2, 24, 9, 11), 40, 1, 1, (0, 2), "image"),
     ((64, 64, 56, 56), 64, 1, 1, 0, "image")])
