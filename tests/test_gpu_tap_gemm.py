@@ -3,7 +3,8 @@ image gradient without columns): residue classes of strides 1 and 2, odd and
 even sizes, paddings and dilations of both parities, rectangular kernels,
 channel counts around a tile and a 32-channel block, bf16-exact and general
 tables, with and without the go scale and the STE, contraction splits, and
-a batch whose planes take two passes (past 2 GiB).  The workspace query tells that a shape takes this kernel.
+batches of two passes (planes past 2 GiB, a nearly empty last round).  The
+workspace query tells that a shape takes this kernel.
 
 Bar: the fp64 gradient within rel 1e-5 of the sum of |terms| plus 1e-6, and a
 2-norm error of at most 4e-7 of the result (what one fp32 sum per tap shows).
@@ -79,6 +80,16 @@ def test_tap_gemm(N, C, H, W, Oc, k, s, p, d, splits, table, fused):
     check(N, C, H, W, Oc, k, s, p, d, table, fused)
 
 
+@pytest.mark.parametrize("N,C,H,W,Oc", [(83, 100, 30, 30, 100), (44, 128, 39, 39, 72)])
+def test_tap_gemm_last_round_split(N, C, H, W, Oc):
+    """A nearly empty last round of blocks: its images are a pass of their own,
+    and the workspace holds less than the whole batch's go planes."""
+    g = ops.conv_geom((N, C, H, W), 3, 1, 1, 1)
+    assert L.query("atx_conv_bwd_data_workspace_bytes", g, Oc) < \
+        6 * L.round_up(9 * C, 128) * L.round_up(Oc, 32) + N * H * W * 6 * L.round_up(Oc, 32)
+    check(N, C, H, W, Oc, 3, 1, 1, 1, "general", True)
+
+
 def test_tap_gemm_two_passes():
     """11 images of 1024 x 1024: 2.2 GB of go planes, more than a pass holds;
     the workspace stays under the pass's bound."""
@@ -107,7 +118,7 @@ def test_padded_1x1(N, C, H, W, Oc, p, table, fused):
 @pytest.mark.parametrize("N,C,H,W,Oc,k,s,p,d", [
     (8, 64, 28, 28, 64, 3, 1, 1, 1), (32, 70, 33, 31, 65, 3, 1, 1, 1),
     (8, 128, 33, 31, 64, 3, 2, 1, 1), (64, 130, 34, 30, 64, 3, 2, 2, 2),
-    (16, 128, 40, 38, 64, (2, 3), 2, 0, 1)])
+    (16, 128, 40, 38, 64, (2, 3), 2, 0, 1), (83, 100, 30, 30, 100, 3, 1, 1, 1)])
 def test_non_finite_table_entries_stay_with_their_taps(N, C, H, W, Oc, k, s, p, d, table):
     """A tap adds nothing to the pixels whose output lies outside go, also when
     its factor is infinite or NaN: everything else keeps its finite value."""
@@ -121,7 +132,7 @@ def test_non_finite_table_entries_stay_with_their_taps(N, C, H, W, Oc, k, s, p, 
     tx = torch.arange(256, device="cuda").float() if table == "exact" else \
         torch.randn(256, generator=gen, device="cuda")
     tx[0], tx[1] = float("inf"), float("nan")
-    assert tap_splits(g, Oc)
+    assert N == 83 or tap_splits(g, Oc)
     gx = ops.conv_backward_data(go, wq, tx, g)
     wt = tx[wq.long()].double().t().contiguous()
     for n in (*range(0, N, 7), N - 1):
