@@ -1030,6 +1030,34 @@ int lut_gemm_f32_tiled(const uint16_t* xt, int Rpad, const uint8_t* wt, int Opad
 // Row tiles of 2048 rows in which every wave has rows.
 static int full_row_tiles(int R) { return (int)cdiv(R - (cg::RT - cg::RPW), cg::RT); }
 
+// Time in microseconds of custom_dw_tile_kernel with its tap quads in `chunks`
+// runs of kq: the workgroups on full row tiles, one per CU, in dispatch order,
+// then those of a last tile that lacks rows for some waves, which are cheaper
+// and fill the gaps.  Fitted to 34 sizes (L = 25 to 2809, 0.1 to 10.6 row
+// tiles, 4 to 128 channel tiles) x 7 splits, off by 5% (rms).  Its picks take
+// 9.94 ms over them; the fewest splits that give 256 workgroups 11.10, or 1024
+// workgroups 10.49, since either count leaves a round nearly empty somewhere
+// (10816 rows x 128 channels, 288 quads: 256 and 185 us against 176; 3136 x
+// 512, 128 quads: 108 and 119 against 103; 7200 x 64, 144 quads: 41 and 59
+// against 38).
+static double tile_time(const cg::Params& p, int kq, int chunks) {
+  constexpr int CUS = 256;
+  const int full_r = full_row_tiles(p.R);
+  const int waves = (int)cdiv(p.R - (p.tiles_r - 1) * cg::RT, cg::RPW);
+  const long long full = (long long)full_r * p.tiles_o * chunks;
+  long long part = (long long)(p.tiles_r - full_r) * p.tiles_o * chunks;
+  const double wf = 9.0 + 2.77 * kq, wp = 9.0 + 2.77 * kq * (0.675 + 0.045 * waves);
+  // CUs free from t0, and those with one more full tile from t0 + wf
+  const double t0 = full / CUS * wf;
+  const long long late = full % CUS, early = CUS - late;
+  double end = late ? t0 + wf : t0, te = t0, tl = t0 + wf;
+  while (part > 0) {
+    if (late == 0 || te <= tl) { part -= early; te += wp; end = std::max(end, te); }
+    else { part -= late; tl += wp; end = std::max(end, tl); }
+  }
+  return end;
+}
+
 extern "C" {
 
 int atx_custom_grad_dx(const uint16_t* xt, int Rpad, const uint8_t* wt, int Opad,
@@ -1126,18 +1154,15 @@ static int custom_dw_run(const uint16_t* xt, int Rpad, const uint8_t* wt, int Op
                             zzx);
   ATX_REQUIRE(xt && wt && dy && tabT && workspace, "atx_custom_grad_dw: null operand");
   if (L % 4 != 0 || (long long)Rpad * 16 > 0x7fffffffLL) {
-    // Fewer (row, channel) tiles than CUs: split the tap quads over enough
-    // workgroups to fill them (each workgroup writes its own taps' entries of
-    // the row tile's slice, so no extra reduction).
+    // The tap quads are split over workgroups (each writes its own taps' entries
+    // of the row tile's slice, so no extra reduction) as tile_time() says.
     const long long tiles = (long long)p.tiles_r * p.tiles_o;
-    // With a last row tile that lacks rows for some waves, four times as many:
-    // its cheaper workgroups then fill the tail (3.06 row tiles x 32 channel
-    // tiles: 770 us with 256 or 512 workgroups, 748 with 1024, 769 with 2048).
-    const int target = full_row_tiles(p.R) < p.tiles_r ? 1024 : 256;
-    if (tiles < target && p.nq >= 16) {
-      const int want = (int)std::min<long long>(cdiv(target, tiles), p.nq / 8);
-      p.kq_chunk = (int)cdiv(p.nq, want);
-      p.kchunks = (int)cdiv(p.nq, p.kq_chunk);
+    double best = 0.0;
+    for (int c = 1; c == 1 || (c <= p.nq / 8 && tiles * c <= 4096); ++c) {
+      const int kq = (int)cdiv(p.nq, c), chunks = (int)cdiv(p.nq, kq);
+      if (chunks < c) continue;
+      const double time = tile_time(p, kq, chunks);
+      if (c == 1 || time < best) { best = time; p.kq_chunk = kq; p.kchunks = chunks; }
     }
     const long long blocks = tiles * p.kchunks;
     ATX_REQUIRE(blocks < 0x7fffffffLL, "atx_custom_grad_dw: grid too large");

@@ -22,7 +22,10 @@ pytestmark = pytest.mark.gpu
 # workgroups)
 SHAPES = [(1, 9, 1, 5), (1, 9, 255, 17), (1, 9, 257, 40), (1, 6, 1792, 24), (1, 6, 1793, 24),
           (1, 66, 2049, 20), (1, 130, 2303, 33), (3, 70, 1301, 16), (7, 64, 586, 48),
-          (8, 12, 268, 130), (4, 37, 964, 16), (32, 40, 196, 24), (64, 66, 65, 40)]
+          (8, 12, 268, 130), (4, 37, 964, 16), (32, 40, 196, 24), (64, 66, 65, 40),
+          # many quads: runs of them per workgroup, the last one shorter, on
+          # partial tiles alone, with full ones before them, and on full ones
+          (10, 609, 25, 20), (87, 405, 25, 40), (41, 333, 49, 24)]
 
 
 @pytest.mark.parametrize("shape", SHAPES)
