@@ -16,11 +16,12 @@ def route(shape, Oc, k, s, p, d=1):
     planes = L.round_up(P * 6 * L.round_up(Oc, 32), 256)
     image, columns = 4 * g.N * g.C * g.H * g.W, 4 * K * P
     slices = (0, *range(2, 65))
+    fits = {"tap": (rest - planes) % image == 0 and (rest - planes) // image in slices,
+            "columns": rest % columns == 0 and rest // columns - 1 in slices,
+            "image": rest % image == 0 and rest // image in slices}
+    assert not (fits["tap"] and fits["columns"])         # the sizes tell them apart
     # stride 1: the columns are KH KW images, so they are looked for first
-    return next(name for name, ok in (
-        ("tap", (rest - planes) % image == 0 and (rest - planes) // image in slices),
-        ("columns", rest % columns == 0 and rest // columns - 1 in slices),
-        ("image", rest % image == 0 and rest // image in slices)) if ok)
+    return next(name for name, ok in fits.items() if ok)
 
 
 # (tap GEMM, columns and their fold in us, LRE table)

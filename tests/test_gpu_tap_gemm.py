@@ -25,10 +25,11 @@ def tap_splits(g, Oc):
     weight planes, the go planes and whole partial images, and not columns."""
     K, P = g.C * g.KH * g.KW, g.N * g.OH * g.OW
     rest = L.query("atx_conv_bwd_data_workspace_bytes", g, Oc) - \
-        6 * L.round_up(K, 128) * L.round_up(Oc, 32) - \
-        L.round_up(P * 6 * L.round_up(Oc, 32), 256)
-    images, odd = divmod(rest, 4 * g.N * g.C * g.H * g.W)
-    return max(images, 1) if odd == 0 and images in (0, *range(2, 65)) else None
+        6 * L.round_up(K, 128) * L.round_up(Oc, 32)
+    images, odd = divmod(rest - L.round_up(P * 6 * L.round_up(Oc, 32), 256),
+                         4 * g.N * g.C * g.H * g.W)
+    columns = rest % (4 * K * P) == 0
+    return max(images, 1) if not (odd or columns) and images in (0, *range(2, 65)) else None
 
 
 def check(N, C, H, W, Oc, k, s, p, d, table, fused, seed=0):
