@@ -87,18 +87,21 @@ __device__ __forceinline__ float bf16_rest(float v) {
   return __builtin_isfinite(v) ? r : 0.0f;
 }
 
-// Byte offset of row v in the LUT GEMM's LDS tables (256-byte lines holding
-// row v of four tables; within a table's 64-byte quarter, chunk g of row v
-// sits at position g ^ ((v >> 1) & 3)).
+// Entry of the row-offset operand for LUT index v: the byte offset of row v in
+// the pair-table kernels' LDS tables (256-byte lines holding row v of four
+// tables; within a table's 64-byte quarter, chunk g of row v sits at position
+// g ^ ((v >> 1) & 3)).  The LUT GEMM, whose lines have byte planes instead of
+// chunks, and the kernels that look a table up by v take the high byte alone.
 __device__ __forceinline__ unsigned row_offset(unsigned v) {
   return v * 256u + (((v >> 1) & 3u) << 4);
 }
 
-// Row-offset operand layout of the LUT GEMM: the k-rows come in quads
-// (Kpad = K rounded up to 4 rows); slot s of a quad holds, for row r, tap
-// k = (s & ~3) | (((r >> 2) + s) & 3), so that the GEMM's row group reading
-// quarter ((r >> 2) + s) & 3 at sub-step s finds its tap in slot s.  Taps at
-// or beyond K hold offset 0.
+// Row-offset operand layout: the k-rows come in quads (Kpad = K rounded up to
+// 4 rows); slot s of a quad holds, for row r, tap k = (s & ~3) | (((r >> 2) + s)
+// & 3), so that the row groups of one LDS read pass find different taps, in
+// different quarters of a line, in one slot: the pair-table kernels read slot s
+// at sub-step s; a lane of the LUT GEMM reads one tap, from the slot of its
+// rows.  Taps at or beyond K hold offset 0.
 __host__ __device__ __forceinline__ int operand_tap(int slot, int r) {
   return (slot & ~3) | (((r >> 2) + slot) & 3);
 }

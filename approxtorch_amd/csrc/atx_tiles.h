@@ -1,8 +1,8 @@
-// Device helpers shared by the LDS-table kernels (the LUT GEMM forward and
-// the pair-table gradients): both tile 2048 rows over 8 waves, lane
-// (row group rg = lane / 4, chunk g = lane % 4) owning rows
-// 256 wave + 64 h + 4 rg + m (h, m = 0..3), and read the row-offset operand
-// [Kpad][Rpad] written by the pack / im2col kernels.
+// Device helpers shared by several kernels: block order, buffer descriptors,
+// and the lane layout of the pair-table gradients and the fp32-class LUT GEMM.
+// Those tile 2048 rows over 8 waves, lane (row group rg = lane / 4, chunk g =
+// lane % 4) owning rows 256 wave + 64 h + 4 rg + m (h, m = 0..3), and read the
+// row-offset operand [Kpad][Rpad] written by the pack / im2col kernels.
 #pragma once
 
 #include "atx_internal.h"
@@ -53,19 +53,6 @@ __device__ __forceinline__ void load_x(XRows& x, __amdgpu_buffer_rsrc_t xs, int 
     x.v[h] = __builtin_bit_cast(
         uint2, __builtin_amdgcn_raw_buffer_load_b64(xs, voff,
                                                     soff + 2 * tiles::NRG * tiles::RQ * h, 0));
-}
-
-// Read XOR mask of sub-step S from quad buffer B for a lane with
-// base = (rg << 6) | (g << 4): chunk g in bits 4-5, table quarter
-// (rg + S) & 3 in bits 6-7, the buffer in bit 16.  Formed in place by asm
-// the compiler can neither hoist (four masks kept live across a kernel's
-// main loop cost registers that then spill) nor fold into every address.
-template <int S, int B>
-__device__ __forceinline__ unsigned quarter_mask(unsigned base) {
-  unsigned t;
-  asm volatile("v_add_u32 %0, %1, %2\n\tv_and_b32 %0, %3, %0\n\tv_or_b32 %0, %4, %0"
-               : "=&v"(t) : "n"(S << 6), "v"(base), "n"(0xf0), "n"(B << 16));
-  return t;
 }
 
 }  // namespace atx

@@ -6,13 +6,12 @@
 // gathered through L1 (grad_x) or one column of it staged in shared memory
 // per output (grad_w).
 //
-// Design (LDS-resident expanded tables, the LUT GEMM forward's layout in
-// fp32).  A workgroup (512 threads, 8 waves) owns 2048 rows r = n*L + l; its
+// Design (LDS-resident expanded tables, as the LUT GEMM forward's, in fp32).  A workgroup (512 threads, 8 waves) owns 2048 rows r = n*L + l; its
 // lanes read the forward's row-offset operand xt [Kpad][Rpad] (no im2col of
 // the saved image).  For a tap k and a tile of 16 channels o it builds the
 // expanded table E[v][o] = T[v][wi(o,k)] (256 rows x 16 fp32 = 16 KiB) from
 // the transposed table T^T (column wi contiguous, L2-resident), four tables
-// to an LDS line with the quarter rotation of the forward, so every 16-byte
+// to an LDS line with the quarter rotation of the operand, so every 16-byte
 // read (four channels of one row) is conflict-free.  Lane (rg, g) owns 16
 // rows and channels 4g..4g+3 of the tile; at sub-step s of a quad it handles
 // tap 4j + ((rg + s) & 3) for all its rows (the operand's slot rotation).

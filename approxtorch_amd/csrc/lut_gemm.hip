@@ -85,8 +85,7 @@ static_assert(QTAB == 1 << 16, "quad buffer select is bit 16 of a read address")
 static_assert(OT == 32 && NWAVE == 8, "tile geometry");
 static_assert(TPL * OT * 2 == LINE, "four 64-byte table rows per line");
 
-// K limits for exact int32 partial sums (entries up to 32767 / 65535).
-constexpr int KMAX_I16 = 65536;
+// K limit of exact int32 partial sums (entries up to 65535).
 constexpr int KMAX_U16 = 32768;
 
 struct GemmParams {
@@ -957,7 +956,10 @@ constexpr int PLAN_CUS = 256;
 //   + for S > 1: 3.6 for the reduce launch and S x R*O x 1.31e-6 for writing
 //     and re-reading one int32 partial slice,
 // step = 0.62 (a k-step of a full tile), 0.44 with the upper-half tables
-// (x_upper given: `upper`; the tables' loads and stores halve).  A least-squares
+// (`upper`; the tables' loads and stores halve).  The flag's value is on the
+// device, so every call that passes one (the int8 layers, the GEMM-level ops)
+// is planned as if it were set: for signed operands a plan at most 3% dearer by
+// the model (19 x 675 x 621 -> 83), the same at most sizes.  A least-squares
 // fit to a sweep of (rt, S) over 38 shapes (19 ResNet-50 layers at batch 64, 10
 // ResNet-18 layers at 128, GEMM and small shapes), both table heights: its
 // picks take 13.29 ms over the sweep, the best pair of each shape 13.24, the

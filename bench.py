@@ -1,11 +1,10 @@
 #!/usr/bin/env python3
 """Benchmark of the LUT approximate-multiplier training path on one MI355X.
 
-Default workload (BASELINE.json metric "ResNet-50 224^2 approx-QAT img/s",
-config 4): ResNet-50, batch 64 x [3,224,224] ~ N(0,1), 1000 classes, every conv
-but the first converted to Conv2d_int8 (weight_bits 8) with the perturbed
-int16 LUT and LRE gradient tables; one step = forward, cross-entropy, LRE
-backward, SGD update.  `value` is img/s of the whole job (1 GPU).
+Default workload (c4, the headline metric "ResNet-50 224^2 approx-QAT img/s"):
+ResNet-50, batch 64 x [3,224,224] ~ N(0,1), 1000 classes, every conv but the
+first converted to Conv2d_int8 (weight_bits 8) with the perturbed int16 LUT and
+LRE gradient tables; one step = forward, cross-entropy, LRE backward, SGD update.  `value` is img/s of the whole job (1 GPU).
 
 Also reported:
   roofline      the dominant kernel, the LUT GEMM (lut_gemm_kernel): LUT-MACs
@@ -14,11 +13,9 @@ Also reported:
                 pass of the timed steps, so that the events' host cost stays
                 out of `value`; bound = LDS, one
                 LUT-MAC = one 2-byte table read from LDS, peak = 256 CUs x
-                256 B/clk x 2.4 GHz.  `valu_peak` is the co-bound of one
-                int32 add per LUT-MAC (256 CUs x 64 lanes x 2.4 GHz).  For
-                weight_bits <= 4 (c5) the LUT GEMM is onehot_gemm_kernel on
-                the int8 matrix cores: 64 int8 ops per LUT-MAC against 5000
-                TOP/s.
+                256 B/clk x 2.4 GHz.  For weight_bits <= 4 (c5) the LUT
+                GEMM is onehot_gemm_kernel on the int8 matrix cores: 64 int8
+                ops per LUT-MAC against 5000 TOP/s.
                 `traffic` = HBM bytes per launch measured by rocprofv3 PMC
                 passes (FETCH_SIZE, WRITE_SIZE; run with --calibrate-copy so
                 the same passes see a copy kernel of known size).
@@ -39,7 +36,6 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 LDS_PEAK_GBS = 256 * 256 * 2.4      # GB/s: 256 CUs x 256 B/clk x 2.4 GHz
-VALU_PEAK_GLUT = 256 * 64 * 2.4      # G int32 adds/s: 256 CUs x 64 lanes x 2.4 GHz
 INT8_PEAK_TOPS = 5000.0              # dense int8 MFMA, TOP/s
 COPY_BYTES = 512 << 20               # --calibrate-copy: bytes read and written per copy
 # HBM bytes per LUT GEMM launch come from rocprofv3 --pmc FETCH_SIZE and
@@ -649,8 +645,6 @@ def roofline(timer, dt, workload, narrow=False):
         "frac": round(2 * achieved_glut / LDS_PEAK_GBS, 4),
         **common,
         "algorithmic_bytes_per_launch": round(2 * gemm_macs / max(launches, 1)),
-        "valu_peak_lut_mac_per_s_G": round(VALU_PEAK_GLUT, 1),
-        "valu_frac": round(achieved_glut / VALU_PEAK_GLUT, 4),
     }
 
 

@@ -505,16 +505,19 @@ int atx_conv_bwd_data_col(const float* go, const uint8_t* wq, const float* tx,
                           hipStream_t stream);
 /* Image gradient of the conv: col as above (with the go scale), folded into
  * gx [N,C,H,W] with the per-tensor fake-quant STE fused when mask != NULL:
- * gx = (mask ? g : 0) / max(scale[0], 1e-12).  A 1x1 stride-1 unpadded conv
- * writes gx straight from the GEMM, and so does a conv of two taps or more,
- * strides of 1 or 2 and enough work (an implicit GEMM over (tap, o) on go
- * split into bf16 planes, which the workspace holds; a batch whose planes
- * exceed 2 GiB takes several passes); otherwise the workspace holds col.
- * When the output tiles cannot fill the GPU the contraction is split into
- * partial slices (in the workspace) summed in a fixed order.  The workspace also holds the
- * tx[wq] values as bf16 parts for the matrix cores (the products are the
- * fp32 products to within 2^-20 relative; exact when tx holds bf16 values,
- * as the STE's integers do).  Size: atx_conv_bwd_data_workspace_bytes(g, O),
+ * gx = (mask ? g : 0) / max(scale[0], 1e-12).  A 1x1 stride-1 conv writes gx
+ * straight from the GEMM (with padding, from go's positions inside the image),
+ * and so does a conv of two taps or more, strides of 1 or 2 and enough work
+ * where that is estimated to be faster than the columns (an implicit GEMM over
+ * (tap, o) on go split into bf16 planes, which the workspace holds; a batch
+ * whose planes exceed 2 GiB, or whose last round of blocks would be nearly
+ * empty, takes several passes); otherwise the workspace holds col.  When the
+ * output tiles cannot fill the GPU the contraction is split into partial
+ * slices (in the workspace) summed in a fixed order.  The workspace also holds
+ * the tx[wq] values as bf16 parts for the matrix cores (the products are the
+ * fp32 products to within 2^-20 relative; exact when tx holds bf16 values, as
+ * the STE's integers do).  A tap adds nothing to the pixels whose output lies
+ * outside go, also where tx is not finite.  Size: atx_conv_bwd_data_workspace_bytes(g, O),
  * nonzero whenever O, K and L are.  Replaces the same calls
  * plus the fold and the fake-quant backward (nn/bgemm_int8.py:116-118,
  * csrc/claude/quantization.cu:223-258). */
@@ -659,8 +662,9 @@ int atx_custom_grad_dx_narrow_img(const uint16_t* xt, int Rpad, const uint8_t* w
 }
 #endif
 
-/* Row-offset encoding of LUT index v used by the LUT GEMM's LDS tables
- * (256-byte lines; bits 4-5 carry the chunk swizzle (v >> 1) & 3). */
+/* Row-offset encoding of LUT index v: its row's byte offset in the pair-table
+ * kernels' LDS tables (256-byte lines; bits 4-5 carry the chunk swizzle (v >>
+ * 1) & 3); other kernels take the index from the high byte. */
 static inline unsigned atx_row_offset(unsigned v) {
   return v * 256u + (((v >> 1) & 3u) << 4);
 }
