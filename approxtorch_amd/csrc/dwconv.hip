@@ -556,17 +556,21 @@ dwconv_bwd_data_strip_kernel(const float* __restrict__ go, const uint8_t* __rest
 // reach it: 1.5 lookups per output instead of 9 (stride 1).  RAG: OW is not
 // a multiple of 4.  The block's sum over its threads is a fixed tree.
 // 64 x 144 x 56 x 56, stride 1, int8: 260 us -> 54 us (2.7 TB/s).
-constexpr int DW_RUN = 14;                       // rows of a run
-
-struct DwRuns { int q, classes, runs, strips; long long tasks; int slices, per; };
+struct DwRuns { int q, rows, classes, runs, strips; long long tasks; int slices, per; };
 
 static DwRuns dw_runs(const atx_conv_geom& g) {
   DwRuns r;
   r.q = g.SH == 1 ? g.DH : 1;                    // output rows per step
   r.classes = std::min(r.q, g.OH);               // runs start at rows 0 .. q - 1
-  r.runs = (int)cdiv(cdiv(g.OH, r.q), DW_RUN);   // runs of one class
   r.strips = (g.OW + 3) / 4;
-  r.tasks = (long long)g.N * r.classes * r.runs * r.strips;
+  // rows of a run: 14, or fewer while that leaves CUs without a block (a run's
+  // first rows are looked up for it alone, so long runs are the cheaper ones):
+  // 32 x 36 x 85 x 32 with stride 2, 72 blocks: 41 -> 17 us with runs of 4 rows
+  for (r.rows = 14;; r.rows = (r.rows + 1) / 2) {
+    r.runs = (int)cdiv(cdiv(g.OH, r.q), r.rows); // runs of one class
+    r.tasks = (long long)g.N * r.classes * r.runs * r.strips;
+    if (r.rows <= 4 || cdiv(r.tasks, DW_THREADS) * g.C >= 256) break;
+  }
   // about 2048 blocks in all, each with whole rounds of its threads; with many
   // channels, more (up to 256 slices), so that a thread's chain of sums stays at
   // two rounds (112 outputs) and does not grow with the batch: at 32 x 960 x
@@ -634,8 +638,8 @@ dwconv_bwd_weight_strip_kernel(const float* __restrict__ go, const T* __restrict
       }
     };
     float v[3][NV];
-    int oh = cls + run * DW_RUN * r.q;
-    const int oh1 = min(g.OH, oh + DW_RUN * r.q);
+    int oh = cls + run * r.rows * r.q;
+    const int oh1 = min(g.OH, oh + r.rows * r.q);
     int ih = oh * SW - g.PH;                     // input row of tap row 0
 #pragma unroll
     for (int i = 0; i + M < 3; ++i) load_row(v[i + M], ih + i * DW);

@@ -1,7 +1,7 @@
 """Which way atx_conv_bwd_data goes to an image gradient, told from its
 workspace (a host query, no GPU): the tap GEMM where it measured faster, the
 columns where padding would be most of its work, and no columns for a padded
-1x1 conv."""
+1x1 conv; and how many blocks share a depthwise weight gradient."""
 import pytest
 
 from approxtorch_amd.backend import _lib as L
@@ -44,3 +44,12 @@ def route(shape, Oc, k, s, p, d=1):
     ((64, 64, 56, 56), 64, 1, 1, 0, "image")])
 def test_route(shape, Oc, k, s, p, way):
     assert route(shape, Oc, k, s, p) == way
+
+
+@pytest.mark.parametrize("shape,s,least", [
+    ((32, 36, 85, 32), 2, 256),        # 41 us on 72 blocks, 17 on 288
+    ((64, 144, 56, 56), 1, 2016),      # 14-row runs
+    ((1, 8, 64, 64), 1, 8)])           # no more work to share
+def test_depthwise_weight_gradient_blocks(shape, s, least):
+    g = ops.conv_geom(shape, 3, s, 0 if s == 2 else 1, 1)
+    assert L.query("atx_dwconv_bwd_weight_workspace_bytes", g) // 36 >= least
